@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <type_traits>
@@ -958,6 +959,123 @@ __global__ __launch_bounds__(64 * (WM * WN + ND), 1) void f16_gemm_stream(float 
   }
 #undef F16_STREAM_STEP
 #undef F16_STREAM_MFMA
+}
+
+// ---------------------------------------------------------------------------
+// 256-row tiles (hb_wide_tiles.h): one tile per 8-wave workgroup, both
+// operands as fp16 tile images, the same v_mfma_f32_16x16x32_f16 sequence per
+// output element as f16_gemm_ring, so the same bits.
+// ---------------------------------------------------------------------------
+
+#include "hb_wide_tiles.h"
+
+struct F16Mma {
+  using Frag = hb_f16x8;
+  using Acc = hb_f32x4;
+  static __device__ inline Acc mma(Frag w, Frag a, Acc c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, a, c, 0, 0, 0);
+#else
+    (void)w, (void)a;
+    return c;
+#endif
+  }
+};
+
+// Readout of one wave's FM x FN blocks, the first at (row, col) of the product:
+// fp16 rounding, bias, activation, then row-major stores.  A 16-row x
+// 32-column piece leaves in two stores of 8 whole 128-byte lines: the upper 8
+// lanes of every 16-lane row trade their first-block values for the second
+// block's of the lanes 8 below (DPP), so a lane then holds row lane % 8 (+ 8
+// in the second store) of the piece, columns 16 * (lane / 8 % 2) +
+// 4 * (lane / 16) .. + 3.  Rows past m are dropped by the buffer bound of the
+// tile (tile_row its first row; the whole offset is in the vector operand, as
+// the range check does not cover the scalar one).  n % 32 == 0: a 32-column
+// pair lies wholly inside or wholly past n.
+template <int MODE, int FM, int FN>
+__device__ __attribute__((always_inline)) inline void f16_store_rows(hb_f32x4 (&acc)[FM][FN], float *y,
+                                                                     const float *bias, int m, int n, int tile_row,
+                                                                     int row, int col, int lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(FN % 2 == 0, "column blocks in pairs");
+  typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+  const bool has_bias = bias != nullptr;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      y + (size_t)tile_row * n, 0, (uint32_t)min(kWideRows, m - tile_row) * (uint32_t)n * 4u, 0x00020000);
+  const int scol = 16 * ((lane >> 3) & 1) + 4 * (lane >> 4);
+  const uint32_t vcol = ((uint32_t)(row - tile_row + (lane & 7)) * (uint32_t)n + (uint32_t)(col + scol)) * 4u;
+#pragma unroll
+  for (int jp = 0; jp < FN / 2; ++jp) {
+    const int c0 = col + jp * 32;
+    if (c0 >= n) continue;
+    const float *b = bias + c0 + 4 * (lane >> 4);
+    const hb_f32x4 b0 = has_bias ? (hb_f32x4)(*(const f32x4_a4 *)b) : hb_f32x4{0, 0, 0, 0};
+    const hb_f32x4 b1 = has_bias ? (hb_f32x4)(*(const f32x4_a4 *)(b + 16)) : hb_f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      hb_u32x4 o0, o1, lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o0[e] = f16_out_bits<MODE>(acc[i][2 * jp][e], b0[e], has_bias);
+        o1[e] = f16_out_bits<MODE>(acc[i][2 * jp + 1][e], b1[e], has_bias);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = (uint32_t)__builtin_amdgcn_update_dpp((int)o0[e], (int)o1[e], kDppRowShr8, 0xf, 0xc, false);
+        hi[e] = (uint32_t)__builtin_amdgcn_update_dpp((int)o1[e], (int)o0[e], kDppRowShl8, 0xf, 0x3, false);
+      }
+      const uint32_t at = vcol + (uint32_t)(i * 16) * (uint32_t)n * 4u + (uint32_t)jp * 128u;
+      __builtin_amdgcn_raw_buffer_store_b128(lo, rsrc, at, 0, 2);
+      __builtin_amdgcn_raw_buffer_store_b128(hi, rsrc, at + (uint32_t)n * 32u, 0, 2);
+    }
+  }
+#endif
+}
+
+template <int BN, int S, int D, int MODE>
+__global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_rows(float *__restrict__ y,
+                                                                   const int8_t *__restrict__ aimg,
+                                                                   const int8_t *__restrict__ wpack,
+                                                                   const float *__restrict__ bias, int m, int k, int n,
+                                                                   int tiles_m, int tiles_n) {
+  constexpr int FM = 2, FN = BN / 16;
+  __shared__ __attribute__((aligned(1024))) int8_t lds[S * 2 * FN * kFragBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ablocks = (m + 15) / 16;
+  int tm, tn;
+  xcd_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  hb_f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  wide_rows_loop<F16Mma, FM, FN, S, D>(acc, lds, aimg, (uint32_t)ablocks * (uint32_t)k * 32u, wpack,
+                                       (uint32_t)n * (uint32_t)k * 2u, ablocks, n / 16, tm * 16 + wave * FM, tn * FN,
+                                       k / 32, wave, lane);
+  f16_store_rows<MODE>(acc, y, bias, m, n, tm * kWideRows, tm * kWideRows + wave * 32, tn * BN, lane);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_square(float *__restrict__ y,
+                                                                     const int8_t *__restrict__ aimg,
+                                                                     const int8_t *__restrict__ wpack,
+                                                                     const float *__restrict__ bias, int m, int k,
+                                                                     int n, int tiles_m, int tiles_n) {
+  constexpr int S = 4;
+  __shared__ __attribute__((aligned(1024))) int8_t lds[S * 32 * kFragBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ablocks = (m + 15) / 16;
+  int tm, tn;
+  xcd_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  hb_f32x4 acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  wide_square_loop<F16Mma, S>(acc, lds, aimg, (uint32_t)ablocks * (uint32_t)k * 32u, wpack,
+                              (uint32_t)n * (uint32_t)k * 2u, ablocks, n / 16, tm * 16, tn * 16, k / 32, wave, lane);
+  f16_store_rows<MODE>(acc, y, bias, m, n, tm * kWideRows, tm * kWideRows + (wave / 4) * 128,
+                       tn * 256 + (wave % 4) * 64, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2030,9 +2148,9 @@ bool f16_stream_applies(int m, int k, int n) {
   return 2 * tiles >= cus && (cost < ring_cost || (cost == ring_cost && tiles % cus == 0));
 }
 
-template <int BM, int BN, int S>
-int launch_f16_stream_t(float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n, int mode,
-                        hipStream_t st) {
+int launch_f16_stream(float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n, int mode,
+                      hipStream_t st) {
+  constexpr int BM = kF16StreamBM, BN = kF16StreamBN, S = kF16StreamStages;
   const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
   const int tiles = tiles_m * tiles_n;
   const int grid = std::min(compute_units(), (tiles + 7) / 8 * 8) / 8 * 8;
@@ -2050,18 +2168,78 @@ int launch_f16_stream_t(float *y, const int8_t *a, const int8_t *w, const float 
   return hb_check_launch("f16_gemm_stream");
 }
 
-// Narrow streaming tiles for few rows: 128 x 64 (12 stages of 12 KB) and
-// 256 x 64 (7 stages of 20 KB).  HTP_OPS_AMD_F16_STREAM_SHAPE=2 / 3 selects
-// them wherever the ring path runs (measurement hook); the 256 x 64 form
-// also runs by itself at one 256-row tile (below).
-int f16_stream_narrow() {
-  static const int v = getenv("HTP_OPS_AMD_F16_STREAM_SHAPE") ? atoi(getenv("HTP_OPS_AMD_F16_STREAM_SHAPE")) : 0;
-  return v;
+// One tile per workgroup on 256-row tiles (f16_gemm_rows, f16_gemm_square).
+enum WideTiles { kWideNone = 0, kWide64 = 64, kWide192 = 192, kWide256 = 256 };
+
+// hb_f16_force_wide: -1 automatic, 0 never, else these tiles wherever the ring
+// path writes rows.
+std::atomic<int> g_f16_wide{-1};
+
+bool wide_fits(int m, int k, int n) {
+  const size_t mp = (size_t)((m + 15) / 16 * 16), limit = (size_t)1 << 32;
+  return mp * (size_t)k * 2u < limit && (size_t)n * (size_t)k * 2u < limit && (size_t)kWideRows * (size_t)n * 4u < limit;
 }
 
-int launch_f16_stream(float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n, int mode,
-                      hipStream_t st) {
-  return launch_f16_stream_t<kF16StreamBM, kF16StreamBN, kF16StreamStages>(y, a, w, bias, m, k, n, mode, st);
+// The wide tiles to use, or none: predicted microseconds of every candidate
+// after the image pass, as c + rounds * (a + b * k-steps) + f * (output bytes
+// at 5 TB/s), rounds = tiles on the busiest CU; for the ring shapes, several
+// workgroups to a CU, c + rounds * (a + b * k-steps) + d * k-steps.  Fitted to
+// 83 shapes from 200 to 4173 rows, k 768-8192, n 768-14336 (each kernel forced
+// on each shape; errors 3-5 % on average, 15 % at most).  The choice is within
+// 1 % of the fastest candidate on average, 7 % at most, and against the ring
+// and streaming kernels alone, us before / after: 2048x4096x14336 230 / 202,
+// 4173x1536x6144 108 / 94, 1024x4096x14336 116 / 102, 2048x8192x2048 119 / 89,
+// 4173x8192x2048 221 / 162, 3000x4608x1152 74 / 55, 4096x4096x1024 71 / 58,
+// 1101x2048x8192 61 / 46, 4173x768x3072 39 / 33.  They must lead by 2 %, below
+// which the measurements do not tell them apart.
+WideTiles pick_wide(int m, int k, int n) {
+  const int force = g_f16_wide.load(std::memory_order_relaxed);
+  if (force == 0 || f16_stream_mode() >= 0 || !wide_fits(m, k, n)) return kWideNone;
+  if (force > 0) return (WideTiles)force;
+  const double cus = compute_units(), kt = k / 32, out = (double)m * n * 4.0 / 5e6;
+  auto rounds = [&](int bm, int bn) { return std::ceil((double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus); };
+  auto wide_us = [&](int bm, int bn, double c, double a, double b, double f) {
+    return c + rounds(bm, bn) * (a + b * kt) + f * out;
+  };
+  static const double kRingFit[3][4] = {
+      {13.9, -0.61, 0.4454, -0.2597}, {6.5, 2.40, 0.2598, -0.1467}, {3.7, 0.73, 0.0619, 0.0674}};
+  const int shape = pick_ring_shape(m, n);
+  const double *f = kRingFit[shape];
+  double present = f[0] + rounds(kRingShapes[shape].bm, kRingShapes[shape].bn) * (f[1] + f[2] * kt) + f[3] * kt;
+  if (f16_stream_applies(m, k, n)) present = wide_us(256, 128, 1.75, 5.46, 0.277, 0.90);
+  WideTiles best = kWideNone;
+  double best_us = 0.98 * present;
+  auto consider = [&](WideTiles t, double us) {
+    if (us < best_us) {
+      best_us = us;
+      best = t;
+    }
+  };
+  consider(kWide64, wide_us(256, 64, 2.96, 2.89, 0.209, 1.11));
+  consider(kWide192, wide_us(256, 192, -1.54, 12.96, 0.386, 0.55));
+  consider(kWide256, wide_us(256, 256, -5.23, 16.69, 0.484, 0.53));
+  return best;
+}
+
+template <int MODE>
+int launch_wide_mode(WideTiles wide, float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n,
+                     hipStream_t st) {
+  const int tiles_m = (m + kWideRows - 1) / kWideRows, tiles_n = (n + (int)wide - 1) / (int)wide;
+  const dim3 grid(tiles_m * tiles_n), block(64 * kWideWaves);
+  if (wide == kWide256)
+    hipLaunchKernelGGL((f16_gemm_square<MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
+  else if (wide == kWide192)
+    hipLaunchKernelGGL((f16_gemm_rows<192, 5, 3, MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
+  else
+    hipLaunchKernelGGL((f16_gemm_rows<64, 6, 4, MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
+  return hb_check_launch("f16 256-row tiles");
+}
+
+int launch_wide(WideTiles wide, float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n,
+                int mode, hipStream_t st) {
+  if (mode == 1) return launch_wide_mode<1>(wide, y, a, w, bias, m, k, n, st);
+  if (mode == 2) return launch_wide_mode<2>(wide, y, a, w, bias, m, k, n, st);
+  return launch_wide_mode<0>(wide, y, a, w, bias, m, k, n, st);
 }
 
 int launch_ring(float *y, const float *x, const uint16_t *packed, const float *bias, int m, int k, int n, int channels,
@@ -2072,17 +2250,12 @@ int launch_ring(float *y, const float *x, const uint16_t *packed, const float *b
   hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)ws, x, m, k, mp);
   int rc = hb_check_launch("f16_pack_a");
   if (rc) return rc;
-  // One 256-row tile (193-256 rows): 256 x 64 streaming tiles read the
-  // weights once where they cover half of the CUs (256x4096x14336 70.0 ->
-  // 56.4 us, 256x4096x10240 39.5 -> 37.6; at 192 rows the ring kernel stays
-  // ahead: 192x4096x10240 31.4 against 35.3).
-  // The streaming kernels write row-major rows only; mode 3 takes the ring kernel.
+  // The 256-row-tile and streaming kernels write row-major rows only; mode 3
+  // takes the ring kernel.
   const bool rows_out = mode != 3;
-  const bool narrow_auto = f16_stream_narrow() == 0 && m > 192 && m <= 256 && 2 * ((n + 63) / 64) >= compute_units();
-  if (rows_out && f16_stream_mode() != 0 && (f16_stream_narrow() == 2 || narrow_auto) && k / 32 >= 6)
-    return launch_f16_stream_t<256, 64, 7>(y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
-  if (rows_out && f16_stream_mode() != 0 && f16_stream_narrow() == 3 && k / 32 >= 11)
-    return launch_f16_stream_t<128, 64, 12>(y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
+  const WideTiles wide = rows_out ? pick_wide(m, k, n) : kWideNone;
+  if (wide != kWideNone)
+    return launch_wide(wide, y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
   if (rows_out && f16_stream_applies(m, k, n))
     return launch_f16_stream(y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
   const int shape = pick_ring_shape(m, n);
@@ -2547,6 +2720,12 @@ int hb_f16_force_stream(int setting) {
   const int prev = f16_stream_mode();
   g_f16_stream.store(setting, std::memory_order_relaxed);
   return prev;
+}
+
+int hb_f16_force_wide(int setting) {
+  if (setting != -1 && setting != 0 && setting != kWide64 && setting != kWide192 && setting != kWide256)
+    return hb_invalid("hb_f16_force_wide setting");
+  return g_f16_wide.exchange(setting, std::memory_order_relaxed);
 }
 
 int hb_f16_gemm(float *d_y, const float *d_x, const uint16_t *d_packed, const float *d_bias, int m, int k, int n,

@@ -77,6 +77,7 @@ _SIGNATURES = {
     "hb_w8a8_linear_noalloc": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "hb_w8a8_force_tile": (_c_int, [_c_int]),
     "hb_f16_force_stream": (_c_int, [_c_int]),
+    "hb_f16_force_wide": (_c_int, [_c_int]),
     "hb_f16_force_xstream": (_c_int, [_c_int]),
     "hb_f16_force_splitk": (_c_int, [_c_int]),
     "hb_w8a8_gemm_choice": (_c_int, [_c_int, _c_int, _c_int]),
@@ -358,6 +359,15 @@ def f16_force_stream(setting):
     prev = lib().hb_f16_force_stream(setting)
     if prev < -1:
         check(prev, "hb_f16_force_stream")
+    return prev
+
+
+def f16_force_wide(setting):
+    """Pins the F16 256-row tiles: -1 automatic, 0 never, 64 / 192 / 256 columns
+    wherever the ring path runs; returns the previous setting."""
+    prev = lib().hb_f16_force_wide(setting)
+    if prev < -1:
+        check(prev, "hb_f16_force_wide")
     return prev
 
 

@@ -247,7 +247,8 @@ int hb_f16_gemm(float *d_y, const float *d_x, const uint16_t *d_packed, const fl
 size_t hb_f16_workspace_bytes(int m, int k, int n);
 
 /* Tuning and test hook of the F16 path for 64 rows or more with a workspace:
- * -1 restores the automatic choice (the persistent streaming kernel with
+ * -1 restores the automatic choice (the 256-row tiles of hb_f16_force_wide
+ * where they are predicted fastest, else the persistent streaming kernel with
  * 256 x 128 tiles where they occupy at least half of the CUs and spread more
  * evenly than the ring kernel's, else the one-tile-per-workgroup ring
  * kernel), 0 keeps the ring
@@ -255,6 +256,15 @@ size_t hb_f16_workspace_bytes(int m, int k, int n);
  * Returns the previous setting.  Results are identical either way.  The
  * environment variable HTP_OPS_AMD_F16_STREAM gives the initial value. */
 int hb_f16_force_stream(int setting);
+
+/* Pins the 256-row tiles of the F16 path (one tile of 64, 192 or 256 columns
+ * per workgroup) for 64 rows or more with a workspace, modes 0-2: -1 restores
+ * the automatic choice (a cost model of tiles on the busiest CU, against the
+ * ring and streaming kernels), 0 never, 64 / 192 / 256 those tiles wherever
+ * the ring path runs and hb_f16_force_stream is at its automatic setting.
+ * Returns the previous setting.  Results are identical for every setting.  No
+ * counterpart in the reference. */
+int hb_f16_force_wide(int setting);
 
 /* Pins the activation-streaming F16 kernel (f16_gemm_xstream: the fp32
  * activations read once, converted in registers, for many rows and few

@@ -601,6 +601,50 @@ def test_f16_stream_matches_ring(hip, orc, m, k, n, mode, bias, check_oracle):
         assert_f16_close(got.view(np.float32).reshape(m, n), ref, v_ref, bias_cols, f16_abs_dot(x, w), k)
 
 
+@pytest.mark.parametrize("tiles", [64, 192, 256])
+@pytest.mark.parametrize("m,k,n,mode,bias,check_oracle", [
+    (130, 32, 64, 0, True, True),         # one k-step: fewer than any prefetch depth; most rows past m
+    (257, 64, 96, 1, False, True),        # a second row of tiles with one valid row, n past one column tile
+    (300, 96, 608, 2, True, True),        # an odd number of k-steps, n % 192 == 32
+    (512, 288, 256, 0, False, True),      # nine k-steps: the prefetch depths and their remainders
+    (256, 352, 192, 0, True, False),
+    (700, 544, 2080, 2, True, True),      # 17 k-steps, n % 256 == 32
+    (1029, 1536, 1152, 1, True, False),   # a last tile of 5 rows; long k
+    (4173, 736, 1536, 0, True, False),    # several rounds of tiles, a tile count that the XCDs do not share evenly
+])
+def test_f16_wide_tiles_match_ring(hip, orc, m, k, n, mode, bias, check_oracle, tiles):
+    """The 256-row-tile F16 kernels give the same bits as the ring kernel (the
+    same MFMA sequence per output element) and stay within the F16 bound of
+    the oracle; repeated calls on one workspace agree."""
+    ws = hip.DeviceBuffer(max(hip.f16_workspace_bytes(m, k, n), 2 * ((m + 15) // 16 * 16) * k + 256))
+    x, w, perm, b = f16_case(orc, m, k, n, seed=m + k + n + 11, bias=bias)
+    packed = hip.f16_prepack(hip.DeviceBuffer.from_array(perm), k, n)
+    xd = hip.DeviceBuffer.from_array(x)
+    bd = hip.DeviceBuffer.from_array(b) if bias else None
+    y_wide, y_ring = hip.DeviceBuffer(m * n * 4), hip.DeviceBuffer(m * n * 4)
+    y_wide.fill(0xFF)
+    prev, prev_split, prev_x = hip.f16_force_wide(tiles), hip.f16_force_splitk(0), hip.f16_force_xstream(0)
+    try:
+        for _ in range(3):
+            hip.f16_gemm(y_wide, xd, packed, bd, m, k, n, n, mode, workspace=ws)
+        hip.f16_force_wide(0)
+        stream = hip.f16_force_stream(0)
+        hip.f16_gemm(y_ring, xd, packed, bd, m, k, n, n, mode, workspace=ws)
+        hip.f16_force_stream(stream)
+    finally:
+        hip.f16_force_wide(prev)
+        hip.f16_force_splitk(prev_split)
+        hip.f16_force_xstream(prev_x)
+    hip.sync()
+    got = y_wide.read(np.uint32, m * n)
+    np.testing.assert_array_equal(got, y_ring.read(np.uint32, m * n))
+    if check_oracle:
+        ref = orc.f16_gemm_epilogue(x, perm, b, m, k, n, n, mode)
+        v_ref = orc.f16_gemm_epilogue(x, perm, None, m, k, n, n, 0)
+        bias_cols = np.abs(b)[None, :] if b is not None else 0.0
+        assert_f16_close(got.view(np.float32).reshape(m, n), ref, v_ref, bias_cols, f16_abs_dot(x, w), k)
+
+
 @pytest.mark.parametrize("m,k,n,channels,mode,bias,check_oracle", [
     (4096, 1152, 128, 128, 3, True, True),      # VAE-like: channel-major, one 128-column chunk, 36 k-steps
     (1000, 96, 256, 200, 3, True, True),        # channels < n, three k-steps
