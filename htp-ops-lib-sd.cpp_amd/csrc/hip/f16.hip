@@ -281,27 +281,44 @@ __global__ __launch_bounds__(64 * WM *WN) void f16_gemm_tiles(float *__restrict_
 #include "hb_lds_ring.h"
 static_assert(kFragBytes == kRingTileBytes, "operand tiles are the ring's tiles");
 
+// 16 bytes of the image: 8 values of one row, converted (RNE); rows past m are zeros.
+__device__ inline void pack_slot(uint4 *__restrict__ img, size_t slot, const float *__restrict__ x, int m, int k) {
+  const int kblocks = k / 32;
+  const size_t tile = slot / 64u;
+  const int lane = (int)(slot % 64u);
+  const int mb = (int)(tile / (size_t)kblocks), kb = (int)(tile % (size_t)kblocks);
+  const int row = mb * 16 + (lane & 15);
+  const int k0 = kb * 32 + 8 * (lane >> 4);
+  uint4 out = make_uint4(0u, 0u, 0u, 0u);
+  if (row < m) {
+    const float *xr = x + (size_t)row * k + k0;
+    const hb_f32x4 lo = __builtin_nontemporal_load((const hb_f32x4 *)xr);
+    const hb_f32x4 hi = __builtin_nontemporal_load((const hb_f32x4 *)(xr + 4));
+    const hb_f16x8 h = {(_Float16)lo[0], (_Float16)lo[1], (_Float16)lo[2], (_Float16)lo[3],
+                        (_Float16)hi[0], (_Float16)hi[1], (_Float16)hi[2], (_Float16)hi[3]};
+    out = __builtin_bit_cast(uint4, h);
+  }
+  img[slot] = out;
+}
+
 __global__ __launch_bounds__(256) void f16_pack_a(uint4 *__restrict__ img, const float *__restrict__ x, int m, int k,
                                                  int mp) {
   const size_t slots = (size_t)mp * (size_t)k / 8u;
-  const int kblocks = k / 32;
+  for (size_t slot = (size_t)blockIdx.x * blockDim.x + threadIdx.x; slot < slots;
+       slot += (size_t)gridDim.x * blockDim.x)
+    pack_slot(img, slot, x, m, k);
+}
+
+// Two images in one launch (the parts of a dual QKV request).
+__global__ __launch_bounds__(256) void f16_pack_a2(uint4 *__restrict__ img0, const float *__restrict__ x0, int m0,
+                                                  uint4 *__restrict__ img1, const float *__restrict__ x1, int m1,
+                                                  int k) {
+  const size_t slots0 = (size_t)((m0 + 15) / 16 * 16) * (size_t)k / 8u;
+  const size_t slots = slots0 + (size_t)((m1 + 15) / 16 * 16) * (size_t)k / 8u;
   for (size_t slot = (size_t)blockIdx.x * blockDim.x + threadIdx.x; slot < slots;
        slot += (size_t)gridDim.x * blockDim.x) {
-    const size_t tile = slot / 64u;
-    const int lane = (int)(slot % 64u);
-    const int mb = (int)(tile / (size_t)kblocks), kb = (int)(tile % (size_t)kblocks);
-    const int row = mb * 16 + (lane & 15);
-    const int k0 = kb * 32 + 8 * (lane >> 4);
-    uint4 out = make_uint4(0u, 0u, 0u, 0u);
-    if (row < m) {
-      const float *xr = x + (size_t)row * k + k0;
-      const hb_f32x4 lo = __builtin_nontemporal_load((const hb_f32x4 *)xr);
-      const hb_f32x4 hi = __builtin_nontemporal_load((const hb_f32x4 *)(xr + 4));
-      const hb_f16x8 h = {(_Float16)lo[0], (_Float16)lo[1], (_Float16)lo[2], (_Float16)lo[3],
-                          (_Float16)hi[0], (_Float16)hi[1], (_Float16)hi[2], (_Float16)hi[3]};
-      out = __builtin_bit_cast(uint4, h);
-    }
-    img[slot] = out;
+    if (slot < slots0) pack_slot(img0, slot, x0, m0, k);
+    else pack_slot(img1, slot - slots0, x1, m1, k);
   }
 }
 
@@ -1041,17 +1058,15 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_rows(float *__res
   constexpr int FM = 2, FN = BN / 16;
   __shared__ __attribute__((aligned(1024))) int8_t lds[S * 2 * FN * kFragBytes];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int ablocks = (m + 15) / 16;
   int tm, tn;
   xcd_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const WideOperands o = wide_operands(aimg, m, tm * kWideRows, wpack, n, tn * BN, BN, k / 32);
   hb_f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  wide_rows_loop<F16Mma, FM, FN, S, D>(acc, lds, aimg, (uint32_t)ablocks * (uint32_t)k * 32u, wpack,
-                                       (uint32_t)n * (uint32_t)k * 2u, ablocks, n / 16, tm * 16 + wave * FM, tn * FN,
-                                       k / 32, wave, lane);
+  wide_rows_loop<F16Mma, FM, FN, S, D>(acc, lds, o.a, o.ablocks, o.w, o.wblocks, k / 32, wave, lane);
   f16_store_rows<MODE>(acc, y, bias, m, n, tm * kWideRows, tm * kWideRows + wave * 32, tn * BN, lane);
 }
 
@@ -1064,95 +1079,92 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_square(float *__r
   constexpr int S = 4;
   __shared__ __attribute__((aligned(1024))) int8_t lds[S * 32 * kFragBytes];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int ablocks = (m + 15) / 16;
   int tm, tn;
   xcd_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const WideOperands o = wide_operands(aimg, m, tm * kWideRows, wpack, n, tn * 256, 256, k / 32);
   hb_f32x4 acc[8][4];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  wide_square_loop<F16Mma, S>(acc, lds, aimg, (uint32_t)ablocks * (uint32_t)k * 32u, wpack,
-                              (uint32_t)n * (uint32_t)k * 2u, ablocks, n / 16, tm * 16, tn * 16, k / 32, wave, lane);
+  wide_square_loop<F16Mma, S>(acc, lds, o.a, o.ablocks, o.w, o.wblocks, k / 32, wave, lane);
   f16_store_rows<MODE>(acc, y, bias, m, n, tm * kWideRows, tm * kWideRows + (wave / 4) * 128,
                        tn * 256 + (wave % 4) * 64, lane);
 }
 
 // ---------------------------------------------------------------------------
-// Opcodes 8/10/11/12 with the post-processing in the GEMM epilogue: the ring
-// kernel's 128 x BN tile (whole heads: BN = 192, three heads of 64; BN = 128,
-// one head of 128 or two of 64; all of Q, K or V, since heads * HD is a
-// multiple of BN) is read out to fp16 exactly as f16_gemm_ring reads it out
-// (mode 0, no bias), kept in LDS as fp16 (the values are fp16-exact) instead
-// of going to HBM as f32, and each (32-token tile, head) of it goes through
-// qkv_block, the standalone post-processing kernel's code.  Results are
-// identical to f16_gemm_ring followed by qkv_post.
+// Opcodes 8/10/11/12 with the post-processing in the GEMM epilogue: 256 x BN
+// tiles of f16_gemm_rows (whole heads, all of Q, K or V), whose waves each
+// hold a 32-row token tile of their heads, read out to fp16 exactly as
+// f16_gemm_ring reads it out (mode 0, no bias) and post-processed in registers
+// (qkv_rows_head).  Results are identical to f16_gemm_ring followed by
+// qkv_post.  The two parts of a dual request are one launch (each its own rows
+// of tiles, weights and norms): the few tiles of the shorter part would leave
+// most of the chip idle by themselves.
 // ---------------------------------------------------------------------------
 
-template <int HD, int BN>
-__global__ __launch_bounds__(256) void f16_qkv_ring(uint16_t *__restrict__ q, uint16_t *__restrict__ k,
-                                                    uint16_t *__restrict__ v, const int8_t *__restrict__ aimg,
-                                                    const int8_t *__restrict__ wpack, const float *__restrict__ bias,
-                                                    const float *__restrict__ q_norm,
-                                                    const float *__restrict__ k_norm, const float *__restrict__ pe,
-                                                    int rope_off, int rope_count, int m, int kdim, int n_heads,
-                                                    int token_tiles, int out_tile0) {
-  constexpr int BM = 128, WM = 2, WN = 2, S = 4;
+struct QkvPart {
+  const int8_t *aimg, *wpack;
+  const float *bias, *q_norm, *k_norm;
+  int m, rope_off, out_tile0;
+};
+
+template <int HD, int WHICH, int FN>
+__device__ __attribute__((always_inline)) inline void qkv_rows_store(hb_f32x4 (&acc)[2][FN], uint16_t *dst,
+                                                                     const QkvPart &part, const float *gamma,
+                                                                     const float *pe, int rope_count, int token_tiles,
+                                                                     int head0, int n0, int row, int lane) {
+  // rotary matrices (4 floats per column pair) of this lane's two rows, from its first column pair
+  const float *pr[2] = {nullptr, nullptr};
+  bool rot[2] = {false, false};
+  const int rows = min(32, part.m - row);
+  if (WHICH < 2 && pe) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * i + (lane & 15), token = part.rope_off + row + r;
+      rot[i] = r < rows && token < rope_count;
+      pr[i] = pe + ((size_t)token * (HD / 2) + 2 * (lane >> 4)) * 4u;
+    }
+  }
+  const size_t head_words = (size_t)token_tiles * (HD / 32) * 1024;
+#pragma unroll
+  for (int h = 0; h < FN / (HD / 16); ++h)
+    qkv_rows_head<HD, WHICH, FN>(acc, h, dst + (size_t)(head0 + h) * head_words, part.out_tile0 + row / 32,
+                                 token_tiles, part.bias ? part.bias + n0 : nullptr, gamma, pr, rot, rows, lane);
+}
+
+template <int HD, int BN, int S, int D>
+__global__ __launch_bounds__(64 * kWideWaves, 2) void f16_qkv_rows(uint16_t *__restrict__ q, uint16_t *__restrict__ k,
+                                                                  uint16_t *__restrict__ v, QkvPart part0,
+                                                                  QkvPart part1, const float *__restrict__ pe,
+                                                                  int rope_count, int kdim, int n_heads,
+                                                                  int token_tiles, int bands0, int bands) {
   static_assert(BN % HD == 0, "whole heads per tile");
-  constexpr int WTM = BM / WM, WTN = BN / WN;
-  constexpr int FM = WTM / 16, FN = WTN / 16;
-  constexpr int STAGE = (BM / 16 + BN / 16) * kFragBytes;
-  constexpr int TS = BN + 8;  // halfwords per LDS row of the tile (padded)
-  constexpr int TILE_BYTES = BM * TS * 2;
-  constexpr int NH = BN / HD;                          // heads per tile, post-processed together
-  constexpr int POST_BYTES = TILE_BYTES + NH * HD * 32 * 2;  // the tile, then its packed blocks
-  static_assert(kQkvThreads == 64 * WM * WN, "the post-processing uses the GEMM's 256 threads");
-  __shared__ __attribute__((aligned(1024))) int8_t lds[S * STAGE > POST_BYTES ? S * STAGE : POST_BYTES];
-  uint16_t *blk = (uint16_t *)(lds + TILE_BYTES);
-
-  const int q_cols = n_heads * HD, n = 3 * q_cols;
-  const int tiles_m = (m + BM - 1) / BM, tiles_n = n / BN;
-  int tm, tn;
-  tile_coords_2d<BM, BN>(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  constexpr int FM = 2, FN = BN / 16;
+  __shared__ __attribute__((aligned(1024))) int8_t lds[S * 2 * FN * kFragBytes];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wm = wave / WN, wn = wave % WN;
+  const int q_cols = n_heads * HD, n = 3 * q_cols;
+  int band, tn;
+  xcd_tile(blockIdx.x, bands, n / BN, band, tn);
+  const QkvPart part = band < bands0 ? part0 : part1;
+  const int m0 = (band < bands0 ? band : band - bands0) * kWideRows, n0 = tn * BN;
+  const WideOperands o = wide_operands(part.aimg, part.m, m0, part.wpack, n, n0, BN, kdim / 32);
   hb_f32x4 acc[FM][FN];
-  ring_mainloop<BM, BN, WM, WN, S>(acc, lds, aimg, wpack, m, kdim, n, m0, n0, wave, lane);
-
-  block_barrier();  // every wave is done with the operand stages: LDS holds the tile
-  _Float16 *tile = (_Float16 *)lds;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        tile[(wm * WTM + i * 16 + (lane >> 4) * 4 + r) * TS + wn * WTN + j * 16 + (lane & 15)] =
-            (_Float16)acc[i][j][r];
-  __syncthreads();
+    for (int j = 0; j < FN; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  wide_rows_loop<F16Mma, FM, FN, S, D>(acc, lds, o.a, o.ablocks, o.w, o.wblocks, kdim / 32, wave, lane);
 
+  const int row = m0 + wave * 32;
+  if (row >= part.m) return;
   const int which = n0 / q_cols, head0 = (n0 % q_cols) / HD;
-  uint16_t *dst = which == 0 ? q : which == 1 ? k : v;
-  const int rows_tile = min(BM, m - m0);
-  const size_t head_stride = (size_t)token_tiles * (HD / 32) * 1024;
-  for (int t = 0; t < BM / 32 && 32 * t < rows_tile; ++t) {
-    const int rows = min(32, rows_tile - 32 * t);
-    const int tt = out_tile0 + m0 / 32 + t;
-    const size_t head_base = (size_t)head0 * head_stride;
-    const _Float16 *src = tile + 32 * t * TS;
-    const float *b = bias ? bias + n0 : nullptr;
-    if (which == 0)
-      qkv_blocks<HD, 0, NH>(blk, dst, src, TS, b, q_norm, pe, rope_off, rope_count, rows, m0 + 32 * t, tt,
-                            token_tiles, head_base, head_stride);
-    else if (which == 1)
-      qkv_blocks<HD, 1, NH>(blk, dst, src, TS, b, k_norm, pe, rope_off, rope_count, rows, m0 + 32 * t, tt,
-                            token_tiles, head_base, head_stride);
-    else
-      qkv_blocks<HD, 2, NH>(blk, dst, src, TS, b, nullptr, nullptr, 0, 0, rows, m0 + 32 * t, tt, token_tiles,
-                            head_base, head_stride);
-    __syncthreads();  // the packed blocks' LDS staging is reused by the next token tile
-  }
+  if (which == 0)
+    qkv_rows_store<HD, 0, FN>(acc, q, part, part.q_norm, pe, rope_count, token_tiles, head0, n0, row, lane);
+  else if (which == 1)
+    qkv_rows_store<HD, 1, FN>(acc, k, part, part.k_norm, pe, rope_count, token_tiles, head0, n0, row, lane);
+  else
+    qkv_rows_store<HD, 2, FN>(acc, v, part, nullptr, nullptr, 0, token_tiles, head0, n0, row, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2175,9 +2187,10 @@ enum WideTiles { kWideNone = 0, kWide64 = 64, kWide192 = 192, kWide256 = 256 };
 // path writes rows.
 std::atomic<int> g_f16_wide{-1};
 
-bool wide_fits(int m, int k, int n) {
-  const size_t mp = (size_t)((m + 15) / 16 * 16), limit = (size_t)1 << 32;
-  return mp * (size_t)k * 2u < limit && (size_t)n * (size_t)k * 2u < limit && (size_t)kWideRows * (size_t)n * 4u < limit;
+// 32-bit buffer offsets: a tile's rows of either operand, and of the output.
+bool wide_fits(int k, int n) {
+  const size_t limit = (size_t)1 << 32;
+  return (size_t)kWideRows * (size_t)k * 2u < limit && (size_t)kWideRows * (size_t)n * 4u < limit;
 }
 
 // The wide tiles to use, or none: predicted microseconds of every candidate
@@ -2194,7 +2207,7 @@ bool wide_fits(int m, int k, int n) {
 // which the measurements do not tell them apart.
 WideTiles pick_wide(int m, int k, int n) {
   const int force = g_f16_wide.load(std::memory_order_relaxed);
-  if (force == 0 || f16_stream_mode() >= 0 || !wide_fits(m, k, n)) return kWideNone;
+  if (force == 0 || f16_stream_mode() >= 0 || !wide_fits(k, n)) return kWideNone;
   if (force > 0) return (WideTiles)force;
   const double cus = compute_units(), kt = k / 32, out = (double)m * n * 4.0 / 5e6;
   auto rounds = [&](int bm, int bn) { return std::ceil((double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus); };
@@ -2219,6 +2232,17 @@ WideTiles pick_wide(int m, int k, int n) {
   consider(kWide192, wide_us(256, 192, -1.54, 12.96, 0.386, 0.55));
   consider(kWide256, wide_us(256, 256, -5.23, 16.69, 0.484, 0.53));
   return best;
+}
+
+// Columns per tile of f16_qkv_rows for heads of 64: three heads where they
+// divide Q, K and V, unless the busiest CU has less to do with single heads
+// (the same predicted times; without output bytes, the same for both).
+int qkv_tile_cols(int bands, int k, int n, int n_heads) {
+  if (n_heads % 3 != 0) return 64;
+  const double cus = compute_units(), kt = k / 32;
+  const double us192 = std::ceil(bands * (n / 192) / cus) * (12.96 + 0.386 * kt);
+  const double us64 = 4.5 + std::ceil(bands * (n / 64) / cus) * (2.89 + 0.209 * kt);
+  return us64 < us192 ? 64 : 192;
 }
 
 template <int MODE>
@@ -2354,6 +2378,30 @@ int launch_ring_splitk(float *y, const float *x, const uint16_t *packed, const f
   const int eg = (int)((outs + 255) / 256 < 4096 ? (outs + 255) / 256 : 4096);
   hipLaunchKernelGGL(f16_skinny_epilogue, dim3(eg), dim3(256), 0, st, y, part, bias, m, n, channels, mode, used);
   return hb_check_launch("f16_skinny_epilogue");
+}
+
+// Workgroups of the tiled kernel by output size; the split-K paths take over
+// when that grid has no more workgroups than CUs, and for m <= 16, where a
+// tile's rows are mostly padding (measured at k=4096, n=14336: m=1 65 -> 28
+// us; 77x14336x4096: 264 -> 80 us; 64x4096x4096, 256 tiles of 32x32: 40.6 ->
+// 19.7 us).
+long long tiled_workgroups(int m, int n) {
+  const long long big = ((m + 127) / 128) * (long long)((n + 127) / 128);
+  const long long mid = ((m + 63) / 64) * (long long)((n + 63) / 64);
+  const long long small = ((m + 31) / 32) * (long long)((n + 31) / 32);
+  return big >= 256 ? big : mid >= 128 ? mid : small;
+}
+
+// From 33 rows the split-K ring path, except where the ring kernel has more
+// tiles than CUs at 4 GFLOP or more (77x4096x14336: 38.4 against 44.2 us;
+// counted in the ring's own tiles: 256x11520x1280, 80 tiles of 64 x 64, 67.7
+// on the ring against 27.3) and where the one-launch kernel applies to under
+// 12 MB of weights (77x768x3072: 6.7 against 11.1 us, 64x2048x2048 10.4
+// against 11.3).  Measured, us, previous choice / split-K ring: 100x3072x3072
+// 28.6 / 14.4 and 128x3072x3072 28.8 / 15.1 (one launch), 48x2048x8192 20.4 /
+// 17.0 and 77x1280x5120 17.1 / 14.3 (one launch, 13-34 MB of weights).
+bool ring_before_splitk(int m, int k, int n) {
+  return ring_worth_it(m, k, n) && tiled_workgroups(m, n) > compute_units() && ring_tiles(m, n) > compute_units();
 }
 
 // -1 (default): the split-K ring path by the rules of hb_f16_gemm_ws; 0:
@@ -2638,25 +2686,8 @@ int hb_f16_gemm_ws(float *d_y, const float *d_x, const uint16_t *d_packed, const
                          aligned(d_workspace, 256);
   if (splitk_ok && ring_splitk_mode() == 1)
     return launch_ring_splitk(d_y, d_x, d_packed, d_bias, m, k, n, channels, mode, d_workspace, st);
-  // Tiled variant by output size; the split-K paths take over when that grid
-  // has no more workgroups than CUs, and for m <= 16, where a tile's rows are
-  // mostly padding (measured at k=4096, n=14336: m=1 65 -> 28 us;
-  // 77x14336x4096: 264 -> 80 us; 64x4096x4096, 256 tiles of 32x32: 40.6 ->
-  // 19.7 us).
-  const long long big = ((m + 127) / 128) * (long long)((n + 127) / 128);
-  const long long mid = ((m + 63) / 64) * (long long)((n + 63) / 64);
-  const long long small = ((m + 31) / 32) * (long long)((n + 31) / 32);
-  const long long tiled_wgs = big >= 256 ? big : mid >= 128 ? mid : small;
-  // From 33 rows the split-K ring path, except where the ring kernel has
-  // more tiles than CUs at 4 GFLOP or more (77x4096x14336: 38.4 against
-  // 44.2 us; counted in the ring's own tiles: 256x11520x1280, 80 tiles of
-  // 64 x 64, 67.7 on the ring against 27.3) and where the one-launch kernel applies to under 12 MB of
-  // weights (77x768x3072: 6.7 against 11.1 us, 64x2048x2048 10.4 against
-  // 11.3).  Measured, us, previous choice / split-K ring: 100x3072x3072 28.6
-  // / 14.4 and 128x3072x3072 28.8 / 15.1 (one launch), 48x2048x8192 20.4 /
-  // 17.0 and 77x1280x5120 17.1 / 14.3 (one launch, 13-34 MB of weights).
-  const bool ring_here = ring_worth_it(m, k, n) && tiled_wgs > compute_units() && ring_tiles(m, n) > compute_units();
-  const bool splitk_here = splitk_ok && m > 32 && m <= 256 && !ring_here;
+  const long long tiled_wgs = tiled_workgroups(m, n);
+  const bool splitk_here = splitk_ok && m > 32 && m <= 256 && !ring_before_splitk(m, k, n);
   const int cf = aligned(d_y, 16) ? small_cf(m, k, n) : 0;
   if (splitk_here && (!cf || (size_t)n * (size_t)k * 2u >= ((size_t)12 << 20)))
     return launch_ring_splitk(d_y, d_x, d_packed, d_bias, m, k, n, channels, mode, d_workspace, st);
@@ -2688,6 +2719,8 @@ int hb_f16_gemm_ws(float *d_y, const float *d_x, const uint16_t *d_packed, const
   if (d_workspace && ring_worth_it(m, k, n) && workspace_bytes >= a_image_bytes(m, k) && aligned(d_workspace, 256) &&
       aligned(d_y, 16))
     return launch_ring(d_y, d_x, d_packed, d_bias, m, k, n, channels, mode, d_workspace, st);
+  const long long big = ((m + 127) / 128) * (long long)((n + 127) / 128);
+  const long long mid = ((m + 63) / 64) * (long long)((n + 63) / 64);
   if (big >= 256) {
     hipLaunchKernelGGL((f16_gemm_tiles<128, 128, 2, 2>), dim3((int)big), dim3(256), 0, st, d_y, d_x, d_packed, d_bias,
                        m, k, n, channels, mode);
@@ -2695,7 +2728,7 @@ int hb_f16_gemm_ws(float *d_y, const float *d_x, const uint16_t *d_packed, const
     hipLaunchKernelGGL((f16_gemm_tiles<64, 64, 2, 2>), dim3((int)mid), dim3(256), 0, st, d_y, d_x, d_packed, d_bias,
                        m, k, n, channels, mode);
   } else {
-    hipLaunchKernelGGL((f16_gemm_tiles<32, 32, 2, 2>), dim3((int)small), dim3(256), 0, st, d_y, d_x, d_packed, d_bias,
+    hipLaunchKernelGGL((f16_gemm_tiles<32, 32, 2, 2>), dim3((int)tiled_wgs), dim3(256), 0, st, d_y, d_x, d_packed, d_bias,
                        m, k, n, channels, mode);
   }
   return hb_check_launch("f16_gemm_tiles");
@@ -2739,43 +2772,77 @@ size_t hb_qkv_gemm_workspace_bytes(int tokens, int input_dim) {
   return a_image_bytes(tokens, input_dim);
 }
 
+int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_part *parts, int n_parts,
+                      const float *d_pe, int rope_count, int input_dim, int n_heads, int head_dim, int token_tiles,
+                      void *d_workspace, size_t workspace_bytes, hb_stream s) {
+  if (!d_q || !d_k || !d_v || !parts || n_parts < 1 || n_parts > 2 || !d_workspace)
+    return hb_invalid("hb_qkv_gemm null pointer");
+  if (input_dim < 32 || input_dim % 32 || n_heads <= 0 || (head_dim != 64 && head_dim != 128) ||
+      (n_heads * head_dim) % 128 || !wide_fits(input_dim, 32))
+    return hb_invalid("hb_qkv_gemm shape");
+  QkvPart part[2] = {};
+  size_t need = 0, slots = 0;
+  int bands[2] = {0, 0};
+  for (int i = 0; i < n_parts; ++i) {
+    const hb_qkv_part &p = parts[i];
+    if (!p.d_x || !p.d_packed || !p.d_q_norm || !p.d_k_norm) return hb_invalid("hb_qkv_gemm null pointer");
+    if (p.tokens <= 0 || p.out_offset < 0 || p.out_offset % 32 || p.out_offset / 32 + (p.tokens + 31) / 32 > token_tiles)
+      return hb_invalid("hb_qkv_gemm shape");
+    if (!aligned(p.d_x, 16) || !aligned(p.d_packed, 16) || (p.d_bias && !aligned(p.d_bias, 4)))
+      return hb_invalid("hb_qkv_gemm alignment");
+    if (p.rope_offset < 0 && n_parts > 1) return hb_invalid("hb_qkv_gemm_parts rope offset");
+    part[i] = {(const int8_t *)d_workspace + need, (const int8_t *)p.d_packed, p.d_bias, p.d_q_norm, p.d_k_norm,
+               p.tokens, p.rope_offset, p.out_offset / 32};
+    bands[i] = (p.tokens + kWideRows - 1) / kWideRows;
+    need += a_image_bytes(p.tokens, input_dim);
+    slots += (size_t)((p.tokens + 15) / 16 * 16) * (size_t)input_dim / 8u;
+  }
+  if (workspace_bytes < need) return hb_invalid("hb_qkv_gemm workspace too small");
+  if (!aligned(d_q, 16) || !aligned(d_k, 16) || !aligned(d_v, 16) || !aligned(d_workspace, 256) ||
+      (d_pe && !aligned(d_pe, 16)))
+    return hb_invalid("hb_qkv_gemm alignment");
+  if (d_pe && (parts[0].rope_offset < 0 || rope_count <= 0)) d_pe = nullptr;  // the reference skips the rotation
+  hipStream_t st = hb_resolve_stream(s);
+  const int pg = (int)((slots + 255) / 256 < 65536 ? (slots + 255) / 256 : 65536);
+  if (n_parts == 2) {
+    hipLaunchKernelGGL(f16_pack_a2, dim3(pg), dim3(256), 0, st, (uint4 *)part[0].aimg, parts[0].d_x, part[0].m,
+                       (uint4 *)part[1].aimg, parts[1].d_x, part[1].m, input_dim);
+  } else {
+    hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)part[0].aimg, parts[0].d_x, part[0].m,
+                       input_dim, (part[0].m + 15) / 16 * 16);
+  }
+  int rc = hb_check_launch("f16_pack_a");
+  if (rc) return rc;
+  const int n = 3 * n_heads * head_dim, all = bands[0] + bands[1];
+  const int bn = head_dim == 128 ? 128 : qkv_tile_cols(all, input_dim, n, n_heads);
+  const dim3 grid(all * (n / bn)), block(64 * kWideWaves);
+  if (bn == 192)
+    hipLaunchKernelGGL((f16_qkv_rows<64, 192, 5, 3>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
+                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+  else if (bn == 64)
+    hipLaunchKernelGGL((f16_qkv_rows<64, 64, 6, 4>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
+                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+  else
+    hipLaunchKernelGGL((f16_qkv_rows<128, 128, 6, 4>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
+                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+  return hb_check_launch("f16_qkv_rows");
+}
+
+int hb_qkv_gemm_unsplit(int tokens, int input_dim, int n_heads, int head_dim) {
+  const int n = 3 * n_heads * head_dim;
+  if (tokens <= 128 || input_dim < 32 || n < 32) return 0;
+  if (ring_splitk_mode() == 0) return 1;
+  if (tokens > 256) return !wide_splitk_shape(tokens, input_dim, n);
+  return ring_splitk_mode() != 1 && ring_before_splitk(tokens, input_dim, n);
+}
+
 int hb_qkv_gemm(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const float *d_x, const uint16_t *d_packed,
                 const float *d_bias, const float *d_q_norm, const float *d_k_norm, const float *d_pe, int rope_offset,
                 int rope_count, int tokens, int input_dim, int n_heads, int head_dim, int token_tiles, int out_offset,
                 void *d_workspace, size_t workspace_bytes, hb_stream s) {
-  if (!d_q || !d_k || !d_v || !d_x || !d_packed || !d_q_norm || !d_k_norm || !d_workspace)
-    return hb_invalid("hb_qkv_gemm null pointer");
-  if (tokens <= 0 || input_dim < 32 || input_dim % 32 || n_heads <= 0 || (head_dim != 64 && head_dim != 128) ||
-      (n_heads * head_dim) % 128 || out_offset < 0 || out_offset % 32 ||
-      out_offset / 32 + (tokens + 31) / 32 > token_tiles)
-    return hb_invalid("hb_qkv_gemm shape");
-  if (workspace_bytes < a_image_bytes(tokens, input_dim)) return hb_invalid("hb_qkv_gemm workspace too small");
-  if (!aligned(d_q, 16) || !aligned(d_k, 16) || !aligned(d_v, 16) || !aligned(d_x, 16) || !aligned(d_packed, 16) ||
-      !aligned(d_workspace, 256) || (d_bias && !aligned(d_bias, 4)) || (d_pe && !aligned(d_pe, 16)))
-    return hb_invalid("hb_qkv_gemm alignment");
-  if (d_pe && (rope_offset < 0 || rope_count <= 0)) d_pe = nullptr;  // the reference skips the rotation
-  hipStream_t st = hb_resolve_stream(s);
-  const int m = tokens, k = input_dim, n = 3 * n_heads * head_dim;
-  const int mp = (m + 15) / 16 * 16;
-  const size_t slots = (size_t)mp * k / 8u;
-  const int pg = (int)((slots + 255) / 256 < 65536 ? (slots + 255) / 256 : 65536);
-  hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)d_workspace, d_x, m, k, mp);
-  int rc = hb_check_launch("f16_pack_a");
-  if (rc) return rc;
-  // 128 x 192 tiles (three heads of 64) where the heads allow, else 128 x 128
-  const int bn = head_dim == 64 && (n_heads * head_dim) % 192 == 0 ? 192 : 128;
-  const int grid = ((m + 127) / 128) * (n / bn);
-  const int8_t *a = (const int8_t *)d_workspace, *w = (const int8_t *)d_packed;
-  if (bn == 192)
-    hipLaunchKernelGGL((f16_qkv_ring<64, 192>), dim3(grid), dim3(256), 0, st, d_q, d_k, d_v, a, w, d_bias, d_q_norm,
-                       d_k_norm, d_pe, rope_offset, rope_count, m, k, n_heads, token_tiles, out_offset / 32);
-  else if (head_dim == 64)
-    hipLaunchKernelGGL((f16_qkv_ring<64, 128>), dim3(grid), dim3(256), 0, st, d_q, d_k, d_v, a, w, d_bias, d_q_norm,
-                       d_k_norm, d_pe, rope_offset, rope_count, m, k, n_heads, token_tiles, out_offset / 32);
-  else
-    hipLaunchKernelGGL((f16_qkv_ring<128, 128>), dim3(grid), dim3(256), 0, st, d_q, d_k, d_v, a, w, d_bias,
-                       d_q_norm, d_k_norm, d_pe, rope_offset, rope_count, m, k, n_heads, token_tiles, out_offset / 32);
-  return hb_check_launch("f16_qkv_ring");
+  const hb_qkv_part part = {d_x, d_packed, d_bias, d_q_norm, d_k_norm, rope_offset, tokens, out_offset};
+  return hb_qkv_gemm_parts(d_q, d_k, d_v, &part, 1, d_pe, rope_count, input_dim, n_heads, head_dim, token_tiles,
+                           d_workspace, workspace_bytes, s);
 }
 
 }  // extern "C"

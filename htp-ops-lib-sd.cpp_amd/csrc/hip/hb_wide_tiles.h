@@ -58,11 +58,25 @@ __device__ inline void wait_scalar_loads() {
 #endif
 }
 
-// acc += rows [row_block0, + 2) x 16 of this wave times columns
-// [col_block0, + FN) x 16 of the tile, over ktc k-steps.  lds: S stages of
-// 2 * FN KB, one stage = two k-steps of weights.  Row and column blocks past
-// the images read the last block (their sums are never stored).  On return
-// every load has landed in this wave, but other waves may still read LDS.
+// Operands of a tile: a and w point at its first 16-row block of activations
+// and 16-column block of weights (blocks of ktc KB), of which ablocks and
+// wblocks (from 1 up to the tile's) lie in the image; blocks past them read
+// the last one (their sums are never stored).
+struct WideOperands {
+  const int8_t *a, *w;
+  int ablocks, wblocks;
+};
+__device__ inline WideOperands wide_operands(const int8_t *aimg, int rows, int tile_row, const int8_t *wimg, int cols,
+                                             int tile_col, int bn, int ktc) {
+  const size_t block = (size_t)ktc * kRingTileBytes;
+  return {aimg + (size_t)(tile_row / 16) * block, wimg + (size_t)(tile_col / 16) * block,
+          min(kWideRows, rows - tile_row + 15) / 16, min(bn, cols - tile_col) / 16};
+}
+
+// acc += rows [wave * FM, + FM) x 16 of the tile times its FN x 16 columns,
+// over ktc k-steps.  lds: S stages of 2 * FN KB, one stage = two k-steps of
+// weights.  On return every load has landed in this wave, but other waves may
+// still read LDS.
 //
 // Per step of two k-steps: multiply the first, wait for the next stage,
 // barrier, issue the loads of a later step, multiply the second.  A wave's
@@ -72,28 +86,28 @@ __device__ inline void wait_scalar_loads() {
 // (which needs D - 1 >= S - 3 activation steps ahead).
 template <class Op, int FM, int FN, int S, int D>
 __device__ __attribute__((always_inline)) inline void wide_rows_loop(typename Op::Acc (&acc)[FM][FN], int8_t *lds,
-                                                                    const int8_t *aimg, uint32_t abytes,
-                                                                    const int8_t *wimg, uint32_t wbytes, int ablocks,
-                                                                    int wblocks, int row_block0, int col_block0,
-                                                                    int ktc, int wave, int lane) {
+                                                                    const int8_t *a, int ablocks, const int8_t *w,
+                                                                    int wblocks, int ktc, int wave, int lane) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using Frag = typename Op::Frag;
   constexpr int NB = 2 * FN, PW = (NB + kWideWaves - 1) / kWideWaves, PWL = NB / kWideWaves;
   constexpr int AL = 2 * FM, STAGE = NB * kRingTileBytes, AHEAD = S > D ? S : D;
   static_assert(S >= 4 && D - 1 >= S - 3 && PWL >= 1 && (S - 3) * (AL + PW) < 64, "load counts");
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)aimg, 0, abytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)wimg, 0, wbytes, 0x00020000);
   const uint32_t l16 = (uint32_t)lane * 16u, row_bytes = (uint32_t)ktc * (uint32_t)kRingTileBytes;
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc((void *)a, 0, (uint32_t)ablocks * row_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc((void *)w, 0, (uint32_t)wblocks * row_bytes, 0x00020000);
   const int steps = (ktc + 1) / 2;
   uint32_t soffa[FM], soffb[PW];
   int sub[PW];  // which of the stage's two k-steps a weight block belongs to
 #pragma unroll
-  for (int i = 0; i < FM; ++i) soffa[i] = (uint32_t)min(row_block0 + i, ablocks - 1) * row_bytes;
+  for (int i = 0; i < FM; ++i) soffa[i] = (uint32_t)min(wave * FM + i, ablocks - 1) * row_bytes;
 #pragma unroll
   for (int i = 0; i < PW; ++i) {
     const int b = min(i * kWideWaves + wave, NB - 1);
     sub[i] = wide_uniform(b / FN);
-    soffb[i] = (uint32_t)min(col_block0 + b % FN, wblocks - 1) * row_bytes;
+    soffb[i] = (uint32_t)min(b % FN, wblocks - 1) * row_bytes;
   }
   const bool full = PW == PWL || wave < NB % kWideWaves;  // this wave loads PW blocks of a stage, else PWL
   Frag fa[D][2][FM], fb[2][FN];
@@ -176,31 +190,29 @@ __device__ __attribute__((always_inline)) inline void wide_rows_loop(typename Op
 #endif
 }
 
-// acc += the 128 x 64 piece (wave / 4, wave % 4) of the 256 x 256 tile whose
-// row and column blocks start at row_block0 and col_block0, over ktc k-steps.
+// acc += the 128 x 64 piece (wave / 4, wave % 4) of the 256 x 256 tile, over
+// ktc k-steps.
 // lds: S stages of 32 KB.  As wide_rows_loop otherwise; 2 of the 8 row blocks
 // of a step are multiplied before its barrier, the reads of the next step's
 // fragments and this wave's four loads go between the products of the others.
 template <class Op, int S>
 __device__ __attribute__((always_inline)) inline void wide_square_loop(typename Op::Acc (&acc)[8][4], int8_t *lds,
-                                                                      const int8_t *aimg, uint32_t abytes,
-                                                                      const int8_t *wimg, uint32_t wbytes, int ablocks,
-                                                                      int wblocks, int row_block0, int col_block0,
-                                                                      int ktc, int wave, int lane) {
+                                                                      const int8_t *a, int ablocks, const int8_t *w,
+                                                                      int wblocks, int ktc, int wave, int lane) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using Frag = typename Op::Frag;
   constexpr int FM = 8, FN = 4, PW = 4, FIRST = 2, PHASES = FM - FIRST, READS = FM + FN;
   constexpr int STAGE = 32 * kRingTileBytes;
   static_assert(S >= 4, "at least one stage in flight behind the awaited one");
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)aimg, 0, abytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)wimg, 0, wbytes, 0x00020000);
   const uint32_t l16 = (uint32_t)lane * 16u, row_bytes = (uint32_t)ktc * (uint32_t)kRingTileBytes;
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc((void *)a, 0, (uint32_t)ablocks * row_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc((void *)w, 0, (uint32_t)wblocks * row_bytes, 0x00020000);
   uint32_t soff[PW];  // blocks wave and wave + 8 of each operand
 #pragma unroll
   for (int i = 0; i < PW; ++i)
-    soff[i] = (uint32_t)(i < 2 ? min(row_block0 + i * 8 + wave, ablocks - 1)
-                               : min(col_block0 + (i - 2) * 8 + wave, wblocks - 1)) *
-              row_bytes;
+    soff[i] = (uint32_t)(i < 2 ? min(i * 8 + wave, ablocks - 1) : min((i - 2) * 8 + wave, wblocks - 1)) * row_bytes;
   Frag fa[2][FM], fb[2][FN];
   const int aoff = (wave / 4) * FM * kRingTileBytes + lane * 16;
   const int boff = (16 + (wave % 4) * FN) * kRingTileBytes + lane * 16;

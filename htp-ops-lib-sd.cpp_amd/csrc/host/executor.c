@@ -869,6 +869,13 @@ static void *qkv_output(const htp_view *v, int slot) {
   return htp_executor_scratch(slot, v->bytes);
 }
 
+/* Whether every input of a part can be read where it lies (aligned_input
+ * makes no copy). */
+static int qkv_part_in_place(const qkv_part *p) {
+  return (((uintptr_t)p->act.dev & 15u) | ((uintptr_t)p->q_norm.dev & 3u) | ((uintptr_t)p->k_norm.dev & 3u) |
+          (p->has_bias ? (uintptr_t)p->bias.dev & 3u : 0u)) == 0;
+}
+
 /* Validated request -> queued GEMM + post-processing for each part.
  * rope: pe view or NULL; rope_count the token bound of the rotation. */
 static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, int rope_count, int input_dim,
@@ -897,17 +904,23 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     if (built) extra_us += (now_seconds() - t0) * 1e6;
   }
 
-  /* A part of 512 tokens or more runs the GEMM with the post-processing in
-   * its epilogue (hb_qkv_gemm: its tiles then fill the CUs); a smaller one
-   * the GEMM into scratch, then hb_qkv_post (same results either way). */
+  /* A part of 512 tokens or more, or one whose product the F16 GEMM would not
+   * split over K (from 129 tokens, so that the results are the same either
+   * way), runs the GEMM with the post-processing in its epilogue; the others
+   * the GEMM into scratch, then hb_qkv_post.  Two fused parts are one launch
+   * where no input needs a realigned copy (those share scratch slots). */
   int fused[2] = {0, 0};
-  size_t ws_max = 0;
+  size_t ws_max = 0, ws_sum = 0;
   for (int i = 0; i < n_parts; ++i) {
-    fused[i] = parts[i].tokens >= 512 && (ncols / 3) % 128 == 0;
+    fused[i] = (ncols / 3) % 128 == 0 &&
+               (parts[i].tokens >= 512 || hb_qkv_gemm_unsplit(parts[i].tokens, input_dim, n_heads, head_dim));
     const size_t b = fused[i] ? hb_qkv_gemm_workspace_bytes(parts[i].tokens, input_dim)
                               : hb_f16_workspace_bytes(parts[i].tokens, input_dim, ncols);
     ws_max = b > ws_max ? b : ws_max;
+    ws_sum += b;
   }
+  const int joint = n_parts == 2 && fused[0] && fused[1] && qkv_part_in_place(&parts[0]) && qkv_part_in_place(&parts[1]);
+  if (joint) ws_max = ws_sum;
   int raw_tokens = 0;
   for (int i = 0; i < n_parts; ++i)
     if (!fused[i] && parts[i].tokens > raw_tokens) raw_tokens = parts[i].tokens;
@@ -929,6 +942,7 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     return -5;
   }
   int hrc = 0;
+  hb_qkv_part joined[2];
   for (int i = 0; i < n_parts && !hrc; ++i) {
     qkv_part *p = &parts[i];
     if (stage_in(&p->act, s) || stage_in(&p->q_norm, s) || stage_in(&p->k_norm, s) ||
@@ -943,6 +957,16 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     if (!x || !qn || !kn || (p->has_bias && !b)) {
       hrc = HB_E_HIP;
       break;
+    }
+    if (joint) {
+      const hb_qkv_part j = {x, (const uint16_t *)packed[i], b, qn, kn, p->rope_offset, p->tokens, p->out_offset};
+      joined[i] = j;
+      if (i == 0) continue;
+      hrc = hb_event_record(ev.e[0], s);
+      if (!hrc)
+        hrc = hb_qkv_gemm_parts(dst[0], dst[1], dst[2], joined, 2, d_pe, rope_count, input_dim, n_heads, head_dim,
+                                token_tiles, ws, ws_max, s);
+      continue;
     }
     if (i == 0) hrc = hb_event_record(ev.e[0], s);
     if (!hrc && fused[i])

@@ -101,6 +101,9 @@ _SIGNATURES = {
     "hb_qkv_post": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_void_p]),
     "hb_qkv_gemm_workspace_bytes": (_c_size_t, [_c_int, _c_int]),
     "hb_qkv_gemm": (_c_int, [_c_void_p] * 9 + [_c_int] * 8 + [_c_void_p, _c_size_t, _c_void_p]),
+    "hb_qkv_gemm_parts": (_c_int, [_c_void_p] * 4 + [_c_int, _c_void_p] + [_c_int] * 5 + [_c_void_p, _c_size_t,
+                                                                                        _c_void_p]),
+    "hb_qkv_gemm_unsplit": (_c_int, [_c_int] * 4),
     "hb_model_aux_ws": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p] + [_c_int] * 9 +
                         [ctypes.c_float, _c_void_p, _c_size_t, _c_void_p]),
 }
@@ -717,6 +720,24 @@ def qkv_gemm(q_dev, k_dev, v_dev, x_dev, packed, bias_dev, q_norm_dev, k_norm_de
     check(lib().hb_qkv_gemm(q_dev.ptr, k_dev.ptr, v_dev.ptr, x_dev.ptr, packed.ptr, b, q_norm_dev.ptr,
                             k_norm_dev.ptr, pe, rope_offset, rope_count, tokens, input_dim, n_heads, head_dim,
                             token_tiles, out_offset, workspace.ptr, workspace.nbytes, stream), "hb_qkv_gemm")
+
+
+class QkvPart(ctypes.Structure):
+    """hb_qkv_part."""
+    _fields_ = [(name, _c_void_p) for name in ("x", "packed", "bias", "q_norm", "k_norm")] + \
+               [(name, _c_int) for name in ("rope_offset", "tokens", "out_offset")]
+
+
+def qkv_gemm_parts(q_dev, k_dev, v_dev, parts, pe_dev, rope_count, input_dim, n_heads, head_dim, token_tiles, workspace,
+                   stream=None):
+    """hb_qkv_gemm_parts: one or two (x, packed, bias or None, q_norm, k_norm,
+    rope_offset, tokens, out_offset) parts in one launch."""
+    arr = (QkvPart * len(parts))(*[QkvPart(x.ptr, w.ptr, b.ptr if b else None, qn.ptr, kn.ptr, off, t, out)
+                                   for x, w, b, qn, kn, off, t, out in parts])
+    pe = pe_dev.ptr if pe_dev else None
+    check(lib().hb_qkv_gemm_parts(q_dev.ptr, k_dev.ptr, v_dev.ptr, ctypes.addressof(arr), len(parts), pe, rope_count,
+                                  input_dim, n_heads, head_dim, token_tiles, workspace.ptr, workspace.nbytes, stream),
+          "hb_qkv_gemm_parts")
 
 
 def matmul_params(out, act, wgt, m, k, n, with_elapsed=False):

@@ -735,6 +735,60 @@ def test_hb_qkv_gemm_bit_exact(hip, orc, tokens, n_heads, hd, rope, bias, offset
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("image,text,n_heads,hd,k,bias,pe_rows", [
+    (256, 2300, 24, 64, 768, True, 2556),   # three heads per tile; a last row tile of 252 rows
+    (160, 300, 24, 64, 256, True, 460),     # one head per tile; partial row tiles in both parts
+    (32, 1, 30, 64, 96, False, 20),         # an odd number of k-steps; one text token; rotation stops inside the image
+    (288, 77, 38, 64, 64, True, 0),         # heads not a multiple of three, no rotation
+    (512, 261, 24, 128, 352, True, 700),    # heads of 128; five rows in the last row tile
+])
+def test_hb_qkv_gemm_parts_equal_gemm_then_post(hip, image, text, n_heads, hd, k, bias, pe_rows):
+    """Two parts in one launch equal, bit for bit, the unsplit product of each
+    part followed by hb_qkv_post (which equals the oracle's), into one output;
+    tiles outside the parts stay as they were."""
+    rng = np.random.default_rng(image + text + k)
+    cols, tiles = 3 * n_heads * hd, (image + text + 31) // 32 + 1
+    size = n_heads * h.qkv_head_elems(tiles, hd)
+    _, _, _, _, pe = post_inputs(32, 1, hd, 5, rope_tokens=image + text)
+    pe_dev = dev(pe) if pe_rows else None
+    parts, want = [], [dev(np.full(size, 0x1234, np.uint16)) for _ in range(3)]
+    prev = h.f16_force_splitk(0), h.f16_force_stream(0)
+    try:
+        for tokens, off in ((image, 0), (text, image)):
+            x = dev(rng.normal(0, 1, (tokens, k)).astype(np.float32))
+            w = h.f16_prepack(dev(h.permute_f16(rng.normal(0, 0.05, (k, cols)).astype(np.float16).view(np.uint16))), k,
+                              cols)
+            b = dev(rng.normal(0, 0.1, cols).astype(np.float32)) if bias else None
+            qn, kn = (dev(rng.uniform(0.5, 1.5, hd).astype(np.float32)) for _ in range(2))
+            parts.append((x, w, b, qn, kn, off, tokens, off))
+            raw = h.DeviceBuffer(tokens * cols * 4)
+            h.f16_gemm(raw, x, w, None, tokens, k, cols, cols, 0)  # no workspace: the tiled or one-launch kernel
+            ws = h.DeviceBuffer(2 * (tokens + 15) // 16 * 16 * k * 2 + 256)
+            if tokens > 128:
+                h.f16_gemm(raw, x, w, None, tokens, k, cols, cols, 0, workspace=ws)
+            h.qkv_post(*want, raw, b, qn, kn, pe_dev, off, pe_rows, tokens, n_heads, hd, tiles, off)
+            h.sync()
+    finally:
+        h.f16_force_splitk(prev[0])
+        h.f16_force_stream(prev[1])
+    got = [dev(np.full(size, 0x1234, np.uint16)) for _ in range(3)]
+    ws = h.DeviceBuffer(h.qkv_gemm_workspace_bytes(image, k) + h.qkv_gemm_workspace_bytes(text, k))
+    for _ in range(2):
+        h.qkv_gemm_parts(*got, parts, pe_dev, pe_rows, k, n_heads, hd, tiles, ws)
+    h.sync()
+    for which, (g, w) in enumerate(zip(got, want)):
+        a, b = g.read(np.uint16, size), w.read(np.uint16, size)
+        if min(image, text) > 128:
+            assert np.array_equal(a, b), (which, int((a != b).sum()))
+        else:
+            # up to 128 rows the reference product may add k in another order:
+            # one ulp of the fp16 readout, 2^-11 relative, then Q / K values up
+            # to about 4 x 1.5 in fp16, whose own rounding adds as much
+            fa, fb = (v.view(np.float16).astype(np.float32) for v in (a, b))
+            assert np.all(np.abs(fa - fb) <= 2 ** -9 * (1.0 + np.abs(fb))), which
+
+
+@pytest.mark.gpu
 def test_hb_qkv_gemm_rejects_bad_arguments(hip):
     x = h.DeviceBuffer(1 << 20)
     ws = h.DeviceBuffer(1 << 20)
