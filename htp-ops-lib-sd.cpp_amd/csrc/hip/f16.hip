@@ -1050,7 +1050,7 @@ __device__ __attribute__((always_inline)) inline void f16_store_rows(hb_f32x4 (&
 }
 
 template <int BN, int S, int D, int MODE>
-__global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_rows(float *__restrict__ y,
+__global__ __launch_bounds__(64 * kWideWaves, BN == 64 ? 4 : 2) void f16_gemm_rows(float *__restrict__ y,
                                                                    const int8_t *__restrict__ aimg,
                                                                    const int8_t *__restrict__ wpack,
                                                                    const float *__restrict__ bias, int m, int k, int n,
@@ -1114,27 +1114,33 @@ __device__ __attribute__((always_inline)) inline void qkv_rows_store(hb_f32x4 (&
                                                                      const QkvPart &part, const float *gamma,
                                                                      const float *pe, int rope_count, int token_tiles,
                                                                      int head0, int n0, int row, int lane) {
-  // rotary matrices (4 floats per column pair) of this lane's two rows, from its first column pair
-  const float *pr[2] = {nullptr, nullptr};
-  bool rot[2] = {false, false};
+  // The rotary matrices (4 floats per column pair) of this lane's rows, read
+  // once for all heads of the tile; a row that is not rotated reads some row's.
+  constexpr int FH = HD / 16;
   const int rows = min(32, part.m - row);
-  if (WHICH < 2 && pe) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = 16 * i + (lane & 15), token = part.rope_off + row + r;
-      rot[i] = r < rows && token < rope_count;
-      pr[i] = pe + ((size_t)token * (HD / 2) + 2 * (lane >> 4)) * 4u;
-    }
-  }
   const size_t head_words = (size_t)token_tiles * (HD / 32) * 1024;
 #pragma unroll
-  for (int h = 0; h < FN / (HD / 16); ++h)
-    qkv_rows_head<HD, WHICH, FN>(acc, h, dst + (size_t)(head0 + h) * head_words, part.out_tile0 + row / 32,
-                                 token_tiles, part.bias ? part.bias + n0 : nullptr, gamma, pr, rot, rows, lane);
+  for (int i = 0; i < 2; ++i) {
+    hb_f32x4 mat[FH][2] = {};
+    bool rot = false;
+    if (WHICH < 2 && pe) {
+      const int r = 16 * i + (lane & 15), token = part.rope_off + row + r;
+      rot = r < rows && token < rope_count;
+      const float *pr = pe + ((size_t)min(token, rope_count - 1) * (HD / 2) + 2 * (lane >> 4)) * 4u;
+#pragma unroll
+      for (int j = 0; j < FH; ++j)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) mat[j][u] = *(const hb_f32x4 *)(pr + (8 * j + u) * 4);
+    }
+#pragma unroll
+    for (int h = 0; h < FN / FH; ++h)
+      qkv_rows_head<HD, WHICH, FN>(acc, i, h, dst + (size_t)(head0 + h) * head_words, part.out_tile0 + row / 32,
+                                   token_tiles, part.bias ? part.bias + n0 : nullptr, gamma, rot, mat, rows, lane);
+  }
 }
 
 template <int HD, int BN, int S, int D>
-__global__ __launch_bounds__(64 * kWideWaves, 2) void f16_qkv_rows(uint16_t *__restrict__ q, uint16_t *__restrict__ k,
+__global__ __launch_bounds__(64 * kWideWaves, BN == 64 ? 4 : 2) void f16_qkv_rows(uint16_t *__restrict__ q, uint16_t *__restrict__ k,
                                                                   uint16_t *__restrict__ v, QkvPart part0,
                                                                   QkvPart part1, const float *__restrict__ pe,
                                                                   int rope_count, int kdim, int n_heads,
@@ -2196,7 +2202,7 @@ bool wide_fits(int k, int n) {
 // The wide tiles to use, or none: predicted microseconds of every candidate
 // after the image pass, as c + rounds * (a + b * k-steps) + f * (output bytes
 // at 5 TB/s), rounds = tiles on the busiest CU; for the ring shapes, several
-// workgroups to a CU, c + rounds * (a + b * k-steps) + d * k-steps.  Fitted to
+// workgroups to a CU (also two of the 256 x 64 tiles), d * k-steps besides.  Fitted to
 // 83 shapes from 200 to 4173 rows, k 768-8192, n 768-14336 (each kernel forced
 // on each shape; errors 3-5 % on average, 15 % at most).  The choice is within
 // 1 % of the fastest candidate on average, 7 % at most, and against the ring
@@ -2211,8 +2217,8 @@ WideTiles pick_wide(int m, int k, int n) {
   if (force > 0) return (WideTiles)force;
   const double cus = compute_units(), kt = k / 32, out = (double)m * n * 4.0 / 5e6;
   auto rounds = [&](int bm, int bn) { return std::ceil((double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus); };
-  auto wide_us = [&](int bm, int bn, double c, double a, double b, double f) {
-    return c + rounds(bm, bn) * (a + b * kt) + f * out;
+  auto wide_us = [&](int bm, int bn, double c, double a, double b, double f, double d = 0.0) {
+    return c + rounds(bm, bn) * (a + b * kt) + f * out + d * kt;
   };
   static const double kRingFit[3][4] = {
       {13.9, -0.61, 0.4454, -0.2597}, {6.5, 2.40, 0.2598, -0.1467}, {3.7, 0.73, 0.0619, 0.0674}};
@@ -2228,20 +2234,23 @@ WideTiles pick_wide(int m, int k, int n) {
       best = t;
     }
   };
-  consider(kWide64, wide_us(256, 64, 2.96, 2.89, 0.209, 1.11));
-  consider(kWide192, wide_us(256, 192, -1.54, 12.96, 0.386, 0.55));
-  consider(kWide256, wide_us(256, 256, -5.23, 16.69, 0.484, 0.53));
+  consider(kWide64, wide_us(256, 64, 6.68, -0.77, 0.220, 1.14, -0.029));
+  consider(kWide192, wide_us(256, 192, -2.11, 13.31, 0.391, 0.61));
+  consider(kWide256, wide_us(256, 256, -5.85, 17.16, 0.490, 0.58));
   return best;
 }
 
 // Columns per tile of f16_qkv_rows for heads of 64: three heads where they
-// divide Q, K and V, unless the busiest CU has less to do with single heads
-// (the same predicted times; without output bytes, the same for both).
+// divide Q, K and V, unless single heads, at the measured time per tile on the
+// busiest CU (two of their workgroups share a CU), are faster.  Measured, us,
+// 64 / 192 columns, 24 heads, input 1536: 256 tokens 21.7 / 37.1, 1500 41.6 /
+// 42.2, 2048 58.2 / 44.4, 3000 74.7 / 82.8, 4096 93.1 / 85.9; the rule takes
+// the faster one there and at inputs of 512 and 3072.
 int qkv_tile_cols(int bands, int k, int n, int n_heads) {
   if (n_heads % 3 != 0) return 64;
   const double cus = compute_units(), kt = k / 32;
-  const double us192 = std::ceil(bands * (n / 192) / cus) * (12.96 + 0.386 * kt);
-  const double us64 = 4.5 + std::ceil(bands * (n / 64) / cus) * (2.89 + 0.209 * kt);
+  const double us192 = std::ceil(bands * (n / 192) / cus) * (12.4 + 0.57 * kt);
+  const double us64 = std::ceil(bands * (n / 64) / cus) * (5.4 + 0.246 * kt);
   return us64 < us192 ? 64 : 192;
 }
 
@@ -2255,7 +2264,7 @@ int launch_wide_mode(WideTiles wide, float *y, const int8_t *a, const int8_t *w,
   else if (wide == kWide192)
     hipLaunchKernelGGL((f16_gemm_rows<192, 5, 3, MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
   else
-    hipLaunchKernelGGL((f16_gemm_rows<64, 6, 4, MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
+    hipLaunchKernelGGL((f16_gemm_rows<64, 5, 3, MODE>), grid, block, 0, st, y, a, w, bias, m, k, n, tiles_m, tiles_n);
   return hb_check_launch("f16 256-row tiles");
 }
 
@@ -2820,7 +2829,7 @@ int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_
     hipLaunchKernelGGL((f16_qkv_rows<64, 192, 5, 3>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
                        rope_count, input_dim, n_heads, token_tiles, bands[0], all);
   else if (bn == 64)
-    hipLaunchKernelGGL((f16_qkv_rows<64, 64, 6, 4>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
+    hipLaunchKernelGGL((f16_qkv_rows<64, 64, 5, 3>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
                        rope_count, input_dim, n_heads, token_tiles, bands[0], all);
   else
     hipLaunchKernelGGL((f16_qkv_rows<128, 128, 6, 4>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,

@@ -202,91 +202,87 @@ __device__ inline uint32_t qkv_pair_lane(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1 /* quad_perm 1,0,3,2 */, 0xf, 0xf, true);
 }
 
-// Head h of the wave's blocks; rows: valid rows of the token tile (others are
-// stored as zeros); base: the head's packed region; rot0 / pe: whether row
-// block i's row is rotated, and its first rotary matrix for this lane's columns.
+// Row block i of head h of the wave's blocks; rows: valid rows of the token
+// tile (others are stored as zeros); base: the head's packed region; rot and
+// m: whether this lane's row is rotated, and its rotary matrices for the
+// lane's column pairs (8 j + 2 * (lane / 16) + q).
 template <int HD, int WHICH, int FN>
-__device__ __attribute__((always_inline)) inline void qkv_rows_head(hb_f32x4 (&acc)[2][FN], int h, uint16_t *base,
-                                                                    int tt, int token_tiles, const float *bias,
-                                                                    const float *gamma, const float *const *pe,
-                                                                    const bool *rot, int rows, int lane) {
+__device__ __attribute__((always_inline)) inline void qkv_rows_head(hb_f32x4 (&acc)[2][FN], int i, int h,
+                                                                    uint16_t *base, int tt, int token_tiles,
+                                                                    const float *bias, const float *gamma, bool rot,
+                                                                    const hb_f32x4 (&m)[HD / 16][2], int rows,
+                                                                    int lane) {
   typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int FH = HD / 16;
   const int g = lane >> 4, r16 = lane & 15;
-  hb_f32x4 b[FH], gm[FH];
+  float v[FH][4];
 #pragma unroll
   for (int j = 0; j < FH; ++j) {
-    b[j] = bias ? (hb_f32x4)(*(const f32x4_a4 *)(bias + h * HD + 16 * j + 4 * g)) : hb_f32x4{0, 0, 0, 0};
-    if (WHICH < 2) gm[j] = *(const f32x4_a4 *)(gamma + 16 * j + 4 * g);
+    const hb_f32x4 b = bias ? (hb_f32x4)(*(const f32x4_a4 *)(bias + h * HD + 16 * j + 4 * g)) : hb_f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[j][e] = __fadd_rn((float)(_Float16)acc[i][h * FH + j][e], b[e]);
   }
+  if (WHICH < 2) {
+    float w[4];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    float v[FH][4];
+    for (int e = 0; e < 4; ++e) {
+      float p[2];  // vector lanes 4 g + e and 16 + 4 g + e: columns 32 apart, in order
 #pragma unroll
-    for (int j = 0; j < FH; ++j)
+      for (int q = 0; q < 2; ++q) {
+        p[q] = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[j][e] = __fadd_rn((float)(_Float16)acc[i][h * FH + j][e], b[j][e]);
-    if (WHICH < 2) {
-      float w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float p[2];  // vector lanes 4 g + e and 16 + 4 g + e: columns 32 apart, in order
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          p[q] = 0.0f;
-#pragma unroll
-          for (int j = q; j < FH; j += 2) p[q] = __fadd_rn(p[q], __fmul_rn(v[j][e], v[j][e]));
-        }
-        w[e] = __fadd_rn(p[1], p[0]);                      // 16 apart
-        w[e] = __fadd_rn(w[e], __shfl_xor(w[e], 32, 64));  // 8 apart
-        w[e] = __fadd_rn(w[e], __shfl_xor(w[e], 16, 64));  // 4 apart
+        for (int j = q; j < FH; j += 2) p[q] = __fadd_rn(p[q], __fmul_rn(v[j][e], v[j][e]));
       }
-      const float sum = __fadd_rn(__fadd_rn(w[3], w[1]), __fadd_rn(w[2], w[0]));
-      const float inv = qkv_rsqrt(__fadd_rn(__fdiv_rn(sum, (float)HD), 1.0e-6f));
+      w[e] = __fadd_rn(p[1], p[0]);                      // 16 apart
+      w[e] = __fadd_rn(w[e], __shfl_xor(w[e], 32, 64));  // 8 apart
+      w[e] = __fadd_rn(w[e], __shfl_xor(w[e], 16, 64));  // 4 apart
+    }
+    const float sum = __fadd_rn(__fadd_rn(w[3], w[1]), __fadd_rn(w[2], w[0]));
+    const float inv = qkv_rsqrt(__fadd_rn(__fdiv_rn(sum, (float)HD), 1.0e-6f));
+#pragma unroll
+    for (int j = 0; j < FH; ++j) {
+      const hb_f32x4 gm = *(const f32x4_a4 *)(gamma + 16 * j + 4 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] = __fmul_rn(__fmul_rn(v[j][e], inv), gm[e]);
+    }
+    if (rot) {
 #pragma unroll
       for (int j = 0; j < FH; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[j][e] = __fmul_rn(__fmul_rn(v[j][e], inv), gm[j][e]);
-      if (rot[i]) {
-#pragma unroll
-        for (int j = 0; j < FH; ++j)
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            const hb_f32x4 m = *(const hb_f32x4 *)(pe[i] + (8 * j + q) * 4);
-            const float x0 = v[j][2 * q], x1 = v[j][2 * q + 1];
-            v[j][2 * q] = __fadd_rn(__fmul_rn(x0, m[0]), __fmul_rn(x1, m[1]));
-            v[j][2 * q + 1] = __fadd_rn(__fmul_rn(x0, m[2]), __fmul_rn(x1, m[3]));
-          }
-      }
+        for (int q = 0; q < 2; ++q) {
+          const float x0 = v[j][2 * q], x1 = v[j][2 * q + 1];
+          v[j][2 * q] = __fadd_rn(__fmul_rn(x0, m[j][q][0]), __fmul_rn(x1, m[j][q][1]));
+          v[j][2 * q + 1] = __fadd_rn(__fmul_rn(x0, m[j][q][2]), __fmul_rn(x1, m[j][q][3]));
+        }
     }
-    const int r = 16 * i + r16;
-    const bool valid = r < rows;
-    uint32_t *words = (uint32_t *)base;
+  }
+  const int r = 16 * i + r16;
+  const bool valid = r < rows;
+  uint32_t *words = (uint32_t *)base;
 #pragma unroll
-    for (int j = 0; j < FH; ++j) {
-      uint32_t c01 = 0, c23 = 0;  // this row's columns 0, 1 and 2, 3 of the block's four
-      if (valid) {
-        c01 = (uint32_t)__half_as_ushort(__float2half_rn(v[j][0])) |
-              (uint32_t)__half_as_ushort(__float2half_rn(v[j][1])) << 16;
-        c23 = (uint32_t)__half_as_ushort(__float2half_rn(v[j][2])) |
-              (uint32_t)__half_as_ushort(__float2half_rn(v[j][3])) << 16;
-      }
-      const int c = 16 * j + 4 * g;  // the lane's first column in the head
-      if (WHICH == 1) {
-        uint32_t *dst = words + (size_t)tt * (HD * 16) + (c >> 6) * 1024 + ((c & 63) >> 1) * 32 + r;
-        dst[0] = c01;
-        dst[32] = c23;
-      } else {
-        // the even row's lane takes columns 0, 1 of both rows, the odd row's 2, 3
-        const bool odd = lane & 1;
-        const uint32_t other = qkv_pair_lane(odd ? c01 : c23);
-        const uint32_t lo = odd ? other : c01, hi = odd ? c23 : other;  // even row, odd row
-        const uint2 out = make_uint2((lo & 0xffffu) | (hi << 16), (lo >> 16) | (hi & 0xffff0000u));
-        const int cc = (c & 31) + (odd ? 2 : 0);
-        const size_t tile = WHICH == 0 ? (size_t)tt * (HD / 32) + (size_t)(c >> 5)
-                                       : (size_t)(c >> 5) * (size_t)token_tiles + (size_t)tt;
-        *(uint2 *)(words + tile * 512 + (r >> 1) * 32 + cc) = out;
-      }
+  for (int j = 0; j < FH; ++j) {
+    uint32_t c01 = 0, c23 = 0;  // this row's columns 0, 1 and 2, 3 of the block's four
+    if (valid) {
+      c01 = (uint32_t)__half_as_ushort(__float2half_rn(v[j][0])) |
+            (uint32_t)__half_as_ushort(__float2half_rn(v[j][1])) << 16;
+      c23 = (uint32_t)__half_as_ushort(__float2half_rn(v[j][2])) |
+            (uint32_t)__half_as_ushort(__float2half_rn(v[j][3])) << 16;
+    }
+    const int c = 16 * j + 4 * g;  // the lane's first column in the head
+    if (WHICH == 1) {
+      uint32_t *dst = words + (size_t)tt * (HD * 16) + (c >> 6) * 1024 + ((c & 63) >> 1) * 32 + r;
+      dst[0] = c01;
+      dst[32] = c23;
+    } else {
+      // the even row's lane takes columns 0, 1 of both rows, the odd row's 2, 3
+      const bool odd = lane & 1;
+      const uint32_t other = qkv_pair_lane(odd ? c01 : c23);
+      const uint32_t lo = odd ? other : c01, hi = odd ? c23 : other;  // even row, odd row
+      const uint2 out = make_uint2((lo & 0xffffu) | (hi << 16), (lo >> 16) | (hi & 0xffff0000u));
+      const int cc = (c & 31) + (odd ? 2 : 0);
+      const size_t tile = WHICH == 0 ? (size_t)tt * (HD / 32) + (size_t)(c >> 5)
+                                     : (size_t)(c >> 5) * (size_t)token_tiles + (size_t)tt;
+      *(uint2 *)(words + tile * 512 + (r >> 1) * 32 + cc) = out;
     }
   }
 }
