@@ -17,6 +17,11 @@ constexpr int kMaxDevices = 16;
 std::mutex g_mutex;
 hipStream_t g_streams[kMaxDevices] = {};
 
+// One thread: the device's constant-rate clock to pinned host memory.
+__global__ void stamp_clock(uint64_t *slot) {
+  __hip_atomic_store(slot, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace
 
 int hb_fail(hipError_t err, const char *what) {
@@ -191,6 +196,20 @@ int hb_event_elapsed_ms(float *ms, hb_event start, hb_event stop) {
   if (ms == nullptr) return hb_invalid("hb_event_elapsed_ms out");
   hipError_t err = hipEventElapsedTime(ms, (hipEvent_t)start, (hipEvent_t)stop);
   return err == hipSuccess ? HB_OK : hb_fail(err, "hipEventElapsedTime");
+}
+
+int hb_stamp(uint64_t *h_slot, hb_stream s) {
+  if (h_slot == nullptr) return hb_invalid("hb_stamp slot");
+  hipLaunchKernelGGL(stamp_clock, dim3(1), dim3(1), 0, hb_resolve_stream(s), h_slot);
+  return hb_check_launch("hb_stamp");
+}
+
+int hb_stamp_khz(void) {
+  int dev = 0, khz = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+    khz = 100000;
+  return khz;
 }
 
 // Stream capture into a HIP graph (relaxed mode: host-side library calls

@@ -89,7 +89,7 @@ static void process_map(struct RequestHeader *r, size_t data_size, uint64_t toke
 void htp_channel_process(htp_backend *backend, struct MessageHeader *msg, size_t capacity, uint64_t token) {
   size_t used = 0;
   if (!message_header_validate_layout(msg, capacity, &used)) return;
-  htp_executor_message_begin();
+  htp_executor_message_begin(msg->n_reqs);
   for (int32_t i = 0; i < msg->n_reqs; ++i) {
     const size_t wire = (size_t)msg->req_offsets[i + 1] - (size_t)msg->req_offsets[i];
     const size_t data_size = wire - sizeof(struct RequestHeader);

@@ -72,7 +72,7 @@ int htp_executor_ensure_device(void);
  * synchronises once, writes their elapsed_us fields, and on a GPU failure
  * overwrites their return codes (`state`, an int32 in the request header)
  * with -5. */
-void htp_executor_message_begin(void);
+void htp_executor_message_begin(int requests);
 int htp_executor_message_request(struct OpComputeRequest *req, size_t req_size, void *state);
 int htp_executor_flush(void);
 int htp_executor_message_end(void);

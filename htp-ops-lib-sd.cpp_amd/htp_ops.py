@@ -55,6 +55,8 @@ _SIGNATURES = {
     "hb_event_record": (_c_int, [_c_void_p, _c_void_p]),
     "hb_event_sync": (_c_int, [_c_void_p]),
     "hb_event_elapsed_ms": (_c_int, [ctypes.POINTER(ctypes.c_float), _c_void_p, _c_void_p]),
+    "hb_stamp": (_c_int, [_c_void_p, _c_void_p]),
+    "hb_stamp_khz": (_c_int, []),
     "hb_graph_begin": (_c_int, [_c_void_p]),
     "hb_graph_end": (_c_int, [ctypes.POINTER(_c_void_p), _c_void_p]),
     "hb_graph_launch": (_c_int, [_c_void_p, _c_void_p]),

@@ -454,3 +454,48 @@ def test_mailbox_device_requests_complete_once_per_message(hip, orc):
     for trio in bufs:
         for b in trio:
             b.free()
+
+
+@pytest.mark.parametrize("device_ratio", [1, 3])
+def test_message_of_many_requests_times_every_one(hip, orc, device_ratio):
+    """More requests than the executor defers or has clock slots for, some of
+    them refused and (device_ratio 3) some with host-resident outputs or
+    misaligned outputs copied after the timed work: every return code, output
+    and elapsed_us field is that of the request by itself."""
+    m, k, n, count = 40, 256, 256, 160
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    blob = h.pack_constants(rng.integers(-127, 128, (n, k), dtype=np.int8), rng.uniform(1e-4, 1e-3, n).astype(np.float32))
+    act, cst = h.RpcBuffer(x.nbytes, device=True), h.RpcBuffer(blob.nbytes, device=True)
+    act.write(x)
+    cst.write(blob)
+    stride = m * n * 4 + 64
+    dev_out, host_out = h.RpcBuffer(stride * count, device=True), h.RpcBuffer(stride * count)
+    reqs, where = [], []
+    for i in range(count):
+        host = device_ratio > 1 and i % device_ratio == 1
+        off = stride * i + (8 if not host and device_ratio > 1 and i % 5 == 0 else 0)  # 8: not 16-byte aligned
+        buf, bad = (host_out if host else dev_out), i % 7 == 3
+        where.append((buf, off, bad))
+        reqs.append((h.REQUEST_TYPE_OP_COMPUTE, h.compute_request(15, h.w8a8_params(
+            (buf.fd, off), (act.fd, 0), (cst.fd, 0), 0 if bad else m, k, n, elapsed=-1))))
+    msg, offs = h.build_message(reqs, 16384)
+    raw = (ctypes.c_uint8 * len(msg)).from_buffer(msg)
+    want = orc.linear(x, blob, k, n).view(np.uint32)
+    for _ in range(2):
+        assert h.lib().htp_ops_execute_message(ctypes.addressof(raw), len(msg)) == 0
+        written = 0
+        for i, (buf, off, bad) in enumerate(where):
+            assert h.request_state(msg, offs, i) == (-1 if bad else 0), i
+            elapsed = struct.unpack_from("<i", h.request_data(msg, offs, i), 4 + 36)[0]
+            if bad:
+                assert elapsed == -1
+                continue
+            assert 0 < elapsed < 100000, (i, elapsed)
+            if i % 11 == 0 or i == count - 1 or off % 16:
+                got = buf.read(np.uint32, m * n, off)
+                np.testing.assert_array_equal(got.reshape(m, n), want)
+                written += 1
+        assert written
+    for b in (act, cst, dev_out, host_out):
+        b.free()
