@@ -24,19 +24,37 @@
 // restatement except at rounding ties.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
 
 #include "hb_internal.h"
 
 namespace {
 
+#include "hb_lds_ring.h"
+
 constexpr int kAuxThreads = 256;
 
+int device_cus() {
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+    v = 256;
+  return v;
+}
+
 // x * sigmoid(z), with the stable sigmoid e/(1+e) for z < 0, e = 2^max(-|z|*log2(e), -126).
+// On these arguments the exponential instruction gives exp2f's bits (every
+// float in [-126, 0]) and one Newton step from the reciprocal instruction
+// gives those of the division (every float in [1, 2]); both checked for all
+// of them.  The library function and the division sequence are about half of
+// the instructions of an element.
 __device__ inline float times_sigmoid(float x, float z) {
   const float neg = fmaxf(__fmul_rn(fabsf(z), -1.4426950408889634f), -126.0f);
-  const float e = exp2f(neg);
-  const float inv = __fdiv_rn(1.0f, __fadd_rn(e, 1.0f));
+  const float e = __builtin_amdgcn_exp2f(neg);
+  const float d = __fadd_rn(e, 1.0f), r = __builtin_amdgcn_rcpf(d);
+  const float inv = __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
   return __fmul_rn(x, z < 0.0f ? __fmul_rn(e, inv) : inv);
 }
 
@@ -208,6 +226,7 @@ __global__ __launch_bounds__(T) void aux_norm(float *__restrict__ y, const float
 // cancellation bounded where |mean| >> standard deviation.
 // ws: double sum[tasks][chunks], then double sq[tasks][chunks].
 constexpr int kGnUnroll = 4;
+constexpr int kGnMaxPieces = 64;  // workgroups per group of aux_group_norm_resident
 
 __device__ inline void shifted_add(const float4 v, double shift, double &s, double &q) {
   const double d0 = (double)v.x - shift, d1 = (double)v.y - shift, d2 = (double)v.z - shift,
@@ -225,6 +244,77 @@ __device__ inline unsigned small_quotient(unsigned n, unsigned d, float rd) {
   q += r < 0 ? -1 : (r >= (int)d ? 1 : 0);
   return (unsigned)q;
 }
+
+// The float mean of the reference and 1 / sqrt of its variance from the
+// shifted sums of a whole group.
+__device__ inline void gn_stats(double ts, double tq, int len, float shift, float eps, float *stats) {
+  const double n = (double)len;
+  const float mean = (float)((ts + n * (double)shift) / n);
+  const double e = (double)mean - (double)shift;
+  const double centered = (tq - 2.0 * e * ts) + n * e * e;
+  stats[0] = mean;
+  stats[1] = __fdiv_rn(1.0f, __fsqrt_rn((float)(centered / n + (double)eps)));
+}
+
+// Output of a group's float4s: normalized, affine per channel, activated.
+struct GnOutput {
+  const float *w, *b;
+  float mean, inv, rsp;
+  unsigned pbase, held;  // channels: below 2^31
+  float hw, hb;
+  int spatial, act;
+  bool fast, quad_channel;
+
+  // the same value in every lane, in a scalar register
+  static __device__ inline float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+  }
+
+  __device__ GnOutput(const float *w_, const float *b_, float mean_, float inv_, int task, int channels, int spatial_,
+                      int groups, int act_)
+      : w(w_), b(b_), mean(uniform(mean_)), inv(uniform(inv_)), held(~0u), hw(1.0f), hb(0.0f),
+        spatial(spatial_), act(act_) {
+    const int cpg = channels / groups;
+    pbase = (unsigned)(task % groups) * (unsigned)cpg;
+    rsp = __fdiv_rn(1.0f, (float)spatial);
+    fast = cpg < (1 << 22);  // the channel within the group by small_quotient
+    // spatial % 4 == 0: a quad lies in one channel, and a lane's channel changes
+    // only every spatial / 4 quads, so its parameters stay in registers until then
+    quad_channel = spatial % 4 == 0 && fast;
+  }
+
+  __device__ inline hb_f32x4 value(hb_f32x4 v, int idx) {
+    float o[4] = {v[0], v[1], v[2], v[3]};
+    if (quad_channel && (w || b)) {
+      const unsigned ch = pbase + small_quotient(4u * (unsigned)idx, (unsigned)spatial, rsp);
+      if (ch != held) {
+        held = ch;
+        hw = w ? w[ch] : 1.0f;
+        hb = b ? b[ch] : 0.0f;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float t = __fmul_rn(__fsub_rn(o[e], mean), inv);
+        if (w) t = __fmul_rn(t, hw);
+        if (b) t = __fadd_rn(t, hb);
+        o[e] = act ? activate(t, 4) : t;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float t = __fmul_rn(__fsub_rn(o[e], mean), inv);
+        if (w || b) {
+          const unsigned i = 4u * (unsigned)idx + (unsigned)e;
+          const unsigned ch = pbase + (fast ? small_quotient(i, (unsigned)spatial, rsp) : i / (unsigned)spatial);
+          if (w) t = __fmul_rn(t, w[ch]);
+          if (b) t = __fadd_rn(t, b[ch]);
+        }
+        o[e] = act ? activate(t, 4) : t;
+      }
+    }
+    return hb_f32x4{o[0], o[1], o[2], o[3]};
+  }
+};
 
 template <int PASS>
 __global__ __launch_bounds__(kAuxThreads) void aux_group_norm_chunk(float *__restrict__ y, const float *__restrict__ x,
@@ -266,65 +356,191 @@ __global__ __launch_bounds__(kAuxThreads) void aux_group_norm_chunk(float *__res
       ts += sum[k];
       tq += sq[k];
     }
-    const double n = (double)len;
-    const float mean = (float)((ts + n * (double)shift) / n);
-    const double e = (double)mean - (double)shift;
-    const double centered = (tq - 2.0 * e * ts) + n * e * e;
-    stats[0] = mean;
-    stats[1] = __fdiv_rn(1.0f, __fsqrt_rn((float)(centered / n + (double)eps)));
+    gn_stats(ts, tq, len, shift, eps, stats);
   }
   __syncthreads();
-  const float mean = stats[0], inv = stats[1];
-  const int cpg = channels / groups;
-  const size_t pbase = (size_t)(task % groups) * (size_t)cpg;
-  const float rsp = __fdiv_rn(1.0f, (float)spatial);
-  const bool fast = cpg < (1 << 22);  // the channel within the group by small_quotient
-  // spatial % 4 == 0: a quad lies in one channel, and a lane's channel changes
-  // only every spatial / 4 quads, so its parameters stay in registers until then
-  const bool quad_channel = spatial % 4 == 0 && fast;
-  size_t held = ~(size_t)0;
-  float hw = 1.0f, hb = 0.0f;
-  float4 *yr = (float4 *)(y + offset);
-  auto finish = [&](float4 v, int idx) {
-    float o[4] = {v.x, v.y, v.z, v.w};
-    if (quad_channel && (w || b)) {
-      const size_t ch = pbase + small_quotient(4u * (unsigned)idx, (unsigned)spatial, rsp);
-      if (ch != held) {
-        held = ch;
-        hw = w ? w[ch] : 1.0f;
-        hb = b ? b[ch] : 0.0f;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float t = __fmul_rn(__fsub_rn(o[e], mean), inv);
-        if (w) t = __fmul_rn(t, hw);
-        if (b) t = __fadd_rn(t, hb);
-        o[e] = act ? activate(t, 4) : t;
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float t = __fmul_rn(__fsub_rn(o[e], mean), inv);
-        if (w || b) {
-          const unsigned i = 4u * (unsigned)idx + (unsigned)e;
-          const size_t ch = pbase + (fast ? small_quotient(i, (unsigned)spatial, rsp) : i / (unsigned)spatial);
-          if (w) t = __fmul_rn(t, w[ch]);
-          if (b) t = __fadd_rn(t, b[ch]);
-        }
-        o[e] = act ? activate(t, 4) : t;
-      }
-    }
-    __builtin_nontemporal_store(hb_f32x4{o[0], o[1], o[2], o[3]}, (hb_f32x4 *)(yr + idx));
-  };
+  GnOutput out(w, b, stats[0], stats[1], task, channels, spatial, groups, act);
+  hb_f32x4 *yr = (hb_f32x4 *)(y + offset);
+  const hb_f32x4 *xq = (const hb_f32x4 *)xr;
   int i = v0 + (int)threadIdx.x;
   for (; i + (kGnUnroll - 1) * T < v1; i += kGnUnroll * T) {
-    float4 v[kGnUnroll];
+    hb_f32x4 v[kGnUnroll];
 #pragma unroll
-    for (int u = 0; u < kGnUnroll; ++u) v[u] = xr[i + u * T];
+    for (int u = 0; u < kGnUnroll; ++u) v[u] = xq[i + u * T];
 #pragma unroll
-    for (int u = 0; u < kGnUnroll; ++u) finish(v[u], i + u * T);
+    for (int u = 0; u < kGnUnroll; ++u) __builtin_nontemporal_store(out.value(v[u], i + u * T), yr + i + u * T);
   }
-  for (; i < v1; i += T) finish(xr[i], i);
+  for (; i < v1; i += T) __builtin_nontemporal_store(out.value(xq[i], i), yr + i);
+}
+
+// Group norm over few long groups whose values fit on the chip: x is read
+// once, each workgroup (one per CU) keeping its piece of a group in registers
+// (NV float4 per thread) and LDS (NL float4 per thread) while the group's
+// workgroups exchange the sums of their pieces, then writes the output from
+// there.  Bound by HBM: a second read of x costs as much as the first even
+// where the memory-side cache holds it (aux_group_norm_chunk at 128 channels
+// of 512 x 512: 25 us for the statistics pass and 47 for the output pass, in
+// either order), so 512 KB held per CU save a third of the traffic.  32 groups
+// without parameters, both passes -> this kernel, microseconds: 512 x 128^2
+// 21.4 -> 18.3, 256 x 256^2 39.0 -> 29.4, 256 x 320^2 59.3 -> 44.1, 128 x 512^2
+// 72.2 -> 59.8 (268 MB at 4.5 TB/s; a copy of that size reaches 5.1).
+//
+// The exchange: parts holds one slot per (task, piece, sum) that a fill kernel
+// set to kGnEmpty; every workgroup stores its two sums with device-scope
+// atomics (no fence: a slot is its own flag) and waits for the others' slots.
+// The wait is bounded: if a slot stays empty for spin_ticks of the 100 MHz
+// clock (the other workgroup may not be resident while another kernel holds
+// its CU), the workgroup computes that piece's sums from x itself, the same
+// additions in the same order, so the result does not depend on it and no
+// workgroup ever depends on another to end.  Workgroups of one group run on
+// one XCD where the groups divide by 8 (bid % 8): each XCD then starts whole
+// groups in order.
+//
+// Per thread the sums are added in the order of its pieces' float4s, then as
+// block_sum adds them, then piece by piece in order: fixed for a shape.  The
+// statistics are those of aux_group_norm_chunk.  x and y do not overlap.
+constexpr int kGnThreads = 1024;
+constexpr unsigned long long kGnEmpty = ~0ull;  // a NaN that no sum produces
+
+__global__ void aux_group_norm_clear(unsigned long long *parts, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) parts[i] = kGnEmpty;
+}
+
+__device__ __attribute__((unused)) inline unsigned long long gn_bits(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  return b == kGnEmpty ? 0x7ff8000000000000ull : b;
+}
+
+// Sums over the workgroup, waves in order: thread 0 gets that of s, thread 1
+// that of q.  All threads call it; starts with a barrier.
+__device__ __attribute__((unused)) inline double gn_reduce(double s, double q, double (&red)[2][kGnThreads / 64]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    q += __shfl_xor(q, off, 64);
+  }
+  __syncthreads();  // red and the sums of an earlier call have been read
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s;
+    red[1][threadIdx.x >> 6] = q;
+  }
+  __syncthreads();
+  double total = 0.0;
+  if (threadIdx.x < 2) {
+#pragma unroll 1
+    for (int w = 0; w < kGnThreads / 64; ++w) total += red[threadIdx.x][w];
+  }
+  return total;
+}
+
+template <int NV, int NL>
+__global__ __launch_bounds__(kGnThreads) void aux_group_norm_resident(
+    float *__restrict__ y, const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ b,
+    unsigned long long *parts, int len, int piece, int pieces, int tasks, int channels, int spatial, int groups,
+    float eps, int act, int spin_ticks) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the buffer resource type does not exist in the host pass
+  constexpr int T = kGnThreads;
+  __shared__ float4 held_lds[NL > 0 ? NL * T : 1];
+  __shared__ double red[2][T / 64];
+  __shared__ double sums[2 * kGnMaxPieces];
+  __shared__ float stats[2];
+  const int t = threadIdx.x;
+  int task = blockIdx.x / pieces, mine = blockIdx.x % pieces;
+  if (tasks % 8 == 0) {  // whole groups per XCD
+    const int slot = blockIdx.x / 8;
+    task = blockIdx.x % 8 + 8 * (slot / pieces);
+    mine = slot % pieces;
+  }
+  const size_t offset = (size_t)task * (size_t)len;
+  const float4 *xr = (const float4 *)(x + offset);
+  const int quads = len / 4;
+  const float shift = x[offset];
+  const int v0 = mine * piece, v1 = min(v0 + piece, quads);  // this workgroup's float4s
+
+  // Loads and stores through a buffer resource per row of T float4s (scalar
+  // work): one offset register serves them all, and lanes past the piece read
+  // zeros and store nothing.
+  const int have = max(v1 - v0, 0);
+  const uint32_t at = (uint32_t)t * 16u;
+  auto row = [&](const void *base, int u) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)((const float4 *)base + u * T), 0,
+                                             (uint32_t)max(have - u * T, 0) * 16u, 0x00020000);
+  };
+  const void *xp = xr + v0, *yp = y + offset + 4 * (size_t)v0;
+  // LDS's share straight into LDS, then the registers' (all loads in flight)
+#pragma unroll
+  for (int u = 0; u < NL; ++u)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(row(xp, NV + u), HB_LDS_PTR(held_lds + u * T + (t & ~63)), 16, at, 0, 0,
+                                             0);
+  hb_f32x4 v[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u)
+    v[u] = __builtin_bit_cast(hb_f32x4, __builtin_amdgcn_raw_buffer_load_b128(row(xp, u), at, 0, 0));
+  double s = 0.0, q = 0.0;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    if (u * T + t < have) shifted_add(make_float4(v[u][0], v[u][1], v[u][2], v[u][3]), (double)shift, s, q);
+    __builtin_amdgcn_sched_barrier(0);  // one value's double arithmetic at a time: registers
+  }
+  if (NL > 0) wait_vmcnt<0>();  // this wave's own LDS share has landed
+#pragma unroll
+  for (int u = 0; u < NL; ++u)
+    if ((NV + u) * T + t < have) shifted_add(held_lds[u * T + t], (double)shift, s, q);
+  unsigned long long *slots = parts + (size_t)task * (size_t)pieces * 2u;
+  const double own = gn_reduce(s, q, red);  // thread 0: the sum, thread 1: the squares
+  if (t < 2) __hip_atomic_store(slots + 2 * mine + t, gn_bits(own), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  bool late = false;
+  if (t < 2 * pieces) {
+    unsigned long long bits = kGnEmpty;
+    const uint64_t t0 = wall_clock64();
+    while (bits == kGnEmpty) {
+      bits = __hip_atomic_load(slots + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (bits == kGnEmpty && wall_clock64() - t0 >= (uint64_t)spin_ticks) break;
+      if (bits == kGnEmpty) __builtin_amdgcn_s_sleep(2);
+    }
+    late = bits == kGnEmpty;
+    sums[t] = __longlong_as_double((long long)bits);
+  }
+  if (__syncthreads_or(late)) {
+#pragma unroll 1
+    for (int p = 0; p < pieces; ++p) {
+      const bool missing = (unsigned long long)__double_as_longlong(sums[2 * p]) == kGnEmpty ||
+                           (unsigned long long)__double_as_longlong(sums[2 * p + 1]) == kGnEmpty;
+      if (!missing) continue;  // the same for every thread: sums changes only between the barriers below
+      const int p0 = p * piece, p1 = min(p0 + piece, quads);
+      double ps = 0.0, pq = 0.0;
+#pragma unroll 1
+      for (int i = p0 + t; i < p1; i += T) shifted_add(xr[i], (double)shift, ps, pq);
+      const double total = gn_reduce(ps, pq, red);
+      if (t < 2) sums[2 * p + t] = total;
+      __syncthreads();
+    }
+  }
+  if (t == 0) {
+    double ts = 0.0, tq = 0.0;
+    for (int p = 0; p < pieces; ++p) {
+      ts += sums[2 * p];
+      tq += sums[2 * p + 1];
+    }
+    gn_stats(ts, tq, len, shift, eps, stats);
+  }
+  __syncthreads();
+  GnOutput out(w, b, stats[0], stats[1], task, channels, spatial, groups, act);
+  const int last = quads - 1;  // lanes past the piece compute some value of the group
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const hb_f32x4 o = out.value(v[u], min(v0 + u * T + t, last));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(hb_u32x4, o), row(yp, u), at, 0, 2);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int u = 0; u < NL; ++u) {
+    const float4 l = held_lds[u * T + t];
+    const hb_f32x4 o = out.value(hb_f32x4{l.x, l.y, l.z, l.w}, min(v0 + (NV + u) * T + t, last));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(hb_u32x4, o), row(yp, NV + u), at, 0, 2);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#endif
 }
 
 // Modes 3, 4, 5, 6, 7, 10, 12: one thread per output value, grid-stride.
@@ -522,6 +738,42 @@ GroupPlan group_plan(int tasks, int len) {
   return p;
 }
 
+// The resident form (aux_group_norm_resident): pieces per group so that every
+// group's run at once, one workgroup per CU, and the float4s per thread of a
+// piece; 0 pieces where the values do not fit.
+struct ResidentPlan {
+  int pieces, piece, per_thread;
+};
+// Below 8 M values the two passes are as fast: the second read comes from the
+// XCDs' own L2s, and the exchange costs about 3 us (320 x 128^2, 5.2 M values:
+// 14.3 us in both forms; 512 x 128^2, 8.4 M: 20.1 in two passes, 18.3 here).
+constexpr int64_t kGnResidentMin = 8 << 20;
+constexpr int kGnHeld = 32;  // float4s per thread that registers and LDS hold
+
+ResidentPlan resident_plan(int tasks, int len, int chunks) {
+  ResidentPlan p{0, 0, 0};
+  int pieces = std::min(std::min(device_cus() / tasks, kGnMaxPieces), chunks);
+  if (pieces < 2 || (int64_t)tasks * len < kGnResidentMin) return p;
+  const int quads = len / 4, piece = (quads + pieces - 1) / pieces;
+  if (piece > kGnHeld * kGnThreads) return p;
+  p.pieces = (quads + piece - 1) / piece;
+  p.piece = piece;
+  p.per_thread = (piece + kGnThreads - 1) / kGnThreads;
+  return p;
+}
+
+// How long a workgroup of the resident form waits for another's sums before
+// it computes them itself, in 100 MHz ticks (2 ms; hb_group_norm_spin).
+std::atomic<int> g_gn_spin{200000};
+
+template <int NV, int NL>
+void launch_resident(const ResidentPlan &p, float *y, const float *x, const float *w, const float *b, void *ws, int len,
+                     int tasks, int channels, int spatial, int groups, float eps, int act, hipStream_t st) {
+  hipLaunchKernelGGL((aux_group_norm_resident<NV, NL>), dim3(tasks * p.pieces), dim3(kGnThreads), 0, st, y, x, w, b,
+                     (unsigned long long *)ws, len, p.piece, p.pieces, tasks, channels, spatial, groups, eps, act,
+                     g_gn_spin.load(std::memory_order_relaxed));
+}
+
 int elementwise_grid(int64_t count) {
   const int64_t blocks = (count + kAuxThreads - 1) / kAuxThreads;
   return (int)(blocks < 65536 ? blocks : 65536);
@@ -543,6 +795,11 @@ void launch_elementwise(float *y, const float *x, const float *w, const float *b
 }
 
 }  // namespace
+
+extern "C" int hb_group_norm_spin(int ticks) {
+  if (ticks < 0) return hb_invalid("hb_group_norm_spin ticks");
+  return g_gn_spin.exchange(ticks, std::memory_order_relaxed);
+}
 
 extern "C" size_t hb_model_aux_workspace_bytes(int mode, int channels, int spatial, int groups, int batch) {
   if (mode != 2 || groups <= 0 || channels <= 0 || spatial <= 0 || batch <= 0 || channels % groups) return 0;
@@ -589,6 +846,28 @@ extern "C" int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, c
       if (vec && gp.chunks && d_workspace && workspace_bytes >= need && ((uintptr_t)d_workspace & 7u) == 0) {
         const dim3 grid(gp.chunks, groups * batch);
         double *ws = (double *)d_workspace;
+        const int tasks = groups * batch;
+        const ResidentPlan rp = resident_plan(tasks, len, gp.chunks);
+        const size_t bytes = (size_t)tasks * (size_t)len * 4u;
+        const bool apart = (uintptr_t)d_x + bytes <= (uintptr_t)d_y || (uintptr_t)d_y + bytes <= (uintptr_t)d_x;
+        if (rp.pieces && apart) {
+          const int slots = 2 * tasks * rp.pieces;
+          hipLaunchKernelGGL(aux_group_norm_clear, dim3((slots + 255) / 256), dim3(256), 0, st,
+                             (unsigned long long *)d_workspace, slots);
+          if (int rc = hb_check_launch("aux_group_norm_clear")) return rc;
+          // The fewest registers and the least LDS that hold the piece: 26
+          // float4s take 49.7 us in the largest form and 44.1 in their own
+          // (256 x 320^2), 20 take 43.2 and 39.1 (256 x 80000 values).
+          if (rp.per_thread <= 8)
+            launch_resident<8, 0>(rp, d_y, d_x, d_w, d_b, ws, len, tasks, channels, spatial, groups, eps, activation, st);
+          else if (rp.per_thread <= 16)
+            launch_resident<16, 0>(rp, d_y, d_x, d_w, d_b, ws, len, tasks, channels, spatial, groups, eps, activation, st);
+          else if (rp.per_thread <= 26)
+            launch_resident<20, 6>(rp, d_y, d_x, d_w, d_b, ws, len, tasks, channels, spatial, groups, eps, activation, st);
+          else
+            launch_resident<23, 9>(rp, d_y, d_x, d_w, d_b, ws, len, tasks, channels, spatial, groups, eps, activation, st);
+          break;
+        }
         hipLaunchKernelGGL(aux_group_norm_chunk<0>, grid, block, 0, st, d_y, d_x, d_w, d_b, ws, len, gp.chunk,
                            gp.chunks, groups * batch, channels, spatial, groups, eps, activation);
         hipLaunchKernelGGL(aux_group_norm_chunk<1>, grid, block, 0, st, d_y, d_x, d_w, d_b, ws, len, gp.chunk,

@@ -99,6 +99,7 @@ _SIGNATURES = {
                                 _c_void_p, _c_size_t, _c_void_p]),
     "hb_model_aux": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p] + [_c_int] * 9 + [ctypes.c_float,
                                                                                          _c_void_p]),
+    "hb_group_norm_spin": (_c_int, [_c_int]),
     "hb_model_aux_workspace_bytes": (_c_size_t, [_c_int] * 5),
     "hb_qkv_post": (_c_int, [_c_void_p] * 8 + [_c_int] * 7 + [_c_void_p]),
     "hb_qkv_gemm_workspace_bytes": (_c_size_t, [_c_int, _c_int]),

@@ -329,13 +329,21 @@ int hb_model_aux(float *d_y, const float *d_x, const float *d_w, const float *d_
                  hb_stream s);
 
 /* Workspace for hb_model_aux_ws: nonzero only for group norms (mode 2) with
- * few long groups, which then split each group over many workgroups (three
- * launches; the statistics are added in a fixed order, so the result does not
- * depend on the split).  The workspace holds no state between calls. */
+ * few long groups, which then split each group over many workgroups (two
+ * launches; the statistics are added in an order fixed by the shape).  Groups
+ * of 8 M values or more in all that fit into the CUs' registers and LDS are
+ * read once, if x and y do not overlap.  The workspace holds no state between
+ * calls. */
 size_t hb_model_aux_workspace_bytes(int mode, int channels, int spatial, int groups, int batch);
 int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, const float *d_b, int mode, int count, int width,
                     int channels, int spatial, int groups, int batch, int other_count, int activation, float eps,
                     void *d_workspace, size_t workspace_bytes, hb_stream s);
+
+/* Sets how long (100 MHz ticks, 200000 by default) a workgroup of the
+ * one-read group norm waits for another workgroup's sums before it computes
+ * them itself; returns the previous value.  A test hook: results do not
+ * depend on it. */
+int hb_group_norm_spin(int ticks);
 
 /*
  * Opcodes 8/10/11/12 post-processing (reference src/dsp/ops/mat_mul.c:1051-1371):

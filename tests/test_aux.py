@@ -372,6 +372,66 @@ def test_aux_group_norm_split_gpu(hip, orc, batch, channels, groups, spatial, af
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch,channels,groups,spatial,affine,act,kind", [
+    (1, 512, 32, 16384, True, 1, "normal"),    # 8 M values, the smallest taken: 8 float4 per thread exactly
+    (1, 512, 32, 16388, True, 0, "outlier"),   # one more: the next form, pieces of unequal length
+    (2, 160, 5, 40002, False, 1, "normal"),    # groups that the XCDs do not share evenly; a quad spans two channels
+    (1, 256, 32, 81924, True, 0, "offset"),    # registers and LDS
+    (1, 128, 32, 262140, True, 1, "normal"),   # nearly all that the CUs hold
+    (1, 128, 32, 262148, True, 1, "normal"),   # just past it: two passes
+])
+def test_aux_group_norm_resident_gpu(hip, orc, batch, channels, groups, spatial, affine, act, kind):
+    """Group norm that reads x once, its workgroups exchanging their sums: the
+    oracle's values, and the same bits when no workgroup waits for another
+    (each then computes the missing sums itself) and from call to call."""
+    count = batch * channels * spatial
+    x = rng_normal(count, 160, 2.0) + 0.75
+    if kind == "offset":
+        x = (rng_normal(count, 163, 0.01) + 1000.0).astype(np.float32)
+    elif kind == "outlier":
+        x[::count // (batch * groups)] = 1e4
+    w = rng_normal(channels, 161) if affine else None
+    b = rng_normal(channels, 162) if affine else None
+    kw = dict(mode=2, count=count, width=spatial, channels=channels, spatial=spatial, groups=groups, batch=batch,
+              other_count=channels if affine else 0, activation=act, eps=1e-5)
+    got, init = run_aux(hip, x, w, b, split=True, **kw)
+    again, _ = run_aux(hip, x, w, b, split=True, **kw)
+    prev = hip.lib().hb_group_norm_spin(0)
+    try:
+        alone, _ = run_aux(hip, x, w, b, split=True, **kw)
+    finally:
+        hip.lib().hb_group_norm_spin(prev)
+    assert prev > 0
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    assert np.array_equal(got.view(np.uint32), alone.view(np.uint32))
+    want = orc.model_aux(x, w, b, out=init, **kw)
+    rtol, atol = (ACT_RTOL, ACT_ATOL) if act else (NORM_RTOL, NORM_ATOL)
+    np.testing.assert_allclose(got, want, rtol=rtol, atol=atol)
+
+
+@pytest.mark.gpu
+def test_aux_group_norm_resident_non_finite(hip):
+    """An infinity or a NaN anywhere in a group makes that group NaN (as its
+    mean is) and leaves the others alone; the same in place."""
+    channels, groups, spatial = 512, 32, 16384
+    x = rng_normal(channels * spatial, 170)
+    per = channels // groups * spatial
+    x[3 * per], x[7 * per + 12345], x[9 * per - 1] = np.inf, np.nan, -np.inf
+    kw = dict(mode=2, count=x.size, width=spatial, channels=channels, spatial=spatial, groups=groups, batch=1,
+              other_count=0, activation=0, eps=1e-5)
+    got, _ = run_aux(hip, x, None, None, split=True, **kw)
+    bad = np.isnan(got).reshape(groups, per)
+    assert bad[[3, 7, 8]].all() and not np.delete(bad, [3, 7, 8], 0).any()
+    buf = hip.DeviceBuffer.from_array(x)
+    ws = hip.DeviceBuffer(hip.model_aux_workspace_bytes(2, channels, spatial, groups, 1))
+    hip.model_aux(buf, buf, None, None, workspace=ws, **kw)
+    hip.sync()
+    inplace = buf.read(np.float32, x.size).reshape(groups, per)
+    same = np.delete(np.arange(groups), [3, 7, 8])
+    np.testing.assert_allclose(inplace[same], got.reshape(groups, per)[same], rtol=NORM_RTOL, atol=NORM_ATOL)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", [3, 4])
 @pytest.mark.parametrize("count,other", [(1000, 10), (4096 * 1536, 1536), (12345, 12345)])
 def test_aux_broadcast_gpu(hip, orc, mode, count, other):
