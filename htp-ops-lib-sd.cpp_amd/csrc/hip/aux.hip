@@ -543,28 +543,60 @@ __global__ __launch_bounds__(kGnThreads) void aux_group_norm_resident(
 #endif
 }
 
+// Quotients of indexes below 2^31 by a divisor fixed for the launch: with
+// 2^(s-1) < d <= 2^s and mul = ceil(2^(31+s) / d), n * mul >> (31 + s) is
+// n / d for every n < 2^31 (Granlund and Montgomery, 1994: mul * d exceeds
+// 2^(31+s) by less than 2^s).  A 64-bit division by a kernel argument is
+// about a hundred instructions.
+struct IndexDivisor {
+  uint32_t d, mul, shift;
+
+  __device__ inline uint32_t quotient(uint32_t n) const { return __umulhi(2u * n, mul) >> shift; }
+};
+
+// Divisors past the largest index give 0 for every index, as they should.
+IndexDivisor index_divisor(int64_t d) {
+  IndexDivisor v{(uint32_t)std::min<int64_t>(std::max<int64_t>(d, 1), INT32_MAX), 0, 0};
+  while (((uint64_t)1 << v.shift) < v.d) ++v.shift;
+  v.mul = (uint32_t)((((uint64_t)1 << (31 + v.shift)) + v.d - 1) / v.d);
+  return v;
+}
+
+// Where value i of a mode 3, 4, 10 or 12 finds its other operand: row is the
+// period of w (modes 3, 4) or a row's width, batch the values of a batch.
+struct ElementIndex {
+  IndexDivisor row, batch;
+  uint32_t stride;  // mode 12: values from one row of x to the next
+  bool shared;      // mode 10: one set of parameters for all batches
+
+  template <int MODE>
+  __device__ inline size_t operand(uint32_t i) const {
+    const uint32_t r = row.quotient(i), column = i - r * row.d;
+    if (MODE == 12) return (size_t)r * stride + column;
+    if (MODE == 10 && !shared) return (size_t)batch.quotient(i) * row.d + column;
+    return column;
+  }
+};
+
 // Modes 3, 4, 5, 6, 7, 10, 12: one thread per output value, grid-stride.
 template <int MODE>
 __global__ __launch_bounds__(kAuxThreads) void aux_elementwise(float *__restrict__ y, const float *__restrict__ x,
                                                                const float *__restrict__ w,
                                                                const float *__restrict__ b, int64_t count, int width,
-                                                               int channels, int spatial, int other_count, int act) {
+                                                               ElementIndex at, int act) {
   const int64_t stride = (int64_t)gridDim.x * kAuxThreads;
   for (int64_t i = (int64_t)blockIdx.x * kAuxThreads + threadIdx.x; i < count; i += stride) {
     float v;
     if (MODE == 3) {
-      v = __fadd_rn(x[i], w[i % other_count]);
+      v = __fadd_rn(x[i], w[at.operand<MODE>((uint32_t)i)]);
     } else if (MODE == 4) {
-      v = __fmul_rn(x[i], w[i % other_count]);
+      v = __fmul_rn(x[i], w[at.operand<MODE>((uint32_t)i)]);
     } else if (MODE == 5 || MODE == 6 || MODE == 7) {
       v = activate(x[i], MODE == 5 ? 4 : MODE == 6 ? 1 : 2);
     } else if (MODE == 10) {
-      const int64_t channel = i % width, batch = i / ((int64_t)width * spatial);
-      const int64_t pb = other_count == width ? 0 : batch;
-      v = __fadd_rn(__fmul_rn(x[i], w[pb * width + channel]), b[i]);
+      v = __fadd_rn(__fmul_rn(x[i], w[at.operand<MODE>((uint32_t)i)]), b[i]);
     } else {  // 12
-      const int64_t column = i % width, row = i / width;
-      const float *a = x + row * channels + column;
+      const float *a = x + at.operand<MODE>((uint32_t)i);
       const float gate = a[act ? 0 : width], up = a[act ? width : 0];
       v = __fmul_rn(activate(gate, 5), up);
     }
@@ -572,50 +604,46 @@ __global__ __launch_bounds__(kAuxThreads) void aux_elementwise(float *__restrict
   }
 }
 
-// The same modes, four consecutive values per thread with 16-byte loads and
-// stores (count % 4 == 0, x and y 16-byte aligned; mode 12 also needs width
-// and channels divisible by 4 so each quad of gate and up values is contiguous).
-template <int MODE>
+// The same modes, a quad of consecutive values per thread with 16-byte loads
+// and stores (count % 4 == 0, x and y 16-byte aligned; mode 12 also needs
+// width and channels divisible by 4).  QUAD: the quad's other operand is one
+// 16-byte load too (a row or period of whole quads, aligned), else value by
+// value.  Bound by HBM: one quad per thread keeps the most waves in flight;
+// two or four measured up to 8 % slower (4352 x 1536, mode 6: 11.1 / 12.0 / 12.5
+// us).  Against 64-bit divisions for every value, us: mode 3 40.9 -> 37.8 and
+// mode 10 56.3 -> 54.1 at 4352 x 6144 (5.7 and 5.9 TB/s), 12.7 -> 11.3 and
+// 16.6 -> 15.7 at 4352 x 1536.
+template <int MODE, bool QUAD>
 __global__ __launch_bounds__(kAuxThreads) void aux_elementwise4(float *__restrict__ y, const float *__restrict__ x,
                                                                 const float *__restrict__ w,
-                                                                const float *__restrict__ b, int64_t count4,
-                                                                int width, int channels, int spatial,
-                                                                int other_count, int act) {
-  const int64_t stride = (int64_t)gridDim.x * kAuxThreads;
-  for (int64_t q = (int64_t)blockIdx.x * kAuxThreads + threadIdx.x; q < count4; q += stride) {
-    const int64_t i0 = 4 * q;
-    float o[4];
-    if (MODE == 12) {
-      const int64_t column = i0 % width, row = i0 / width;
-      const float *a = x + row * channels + column;
-      const float4 g = *(const float4 *)(a + (act ? 0 : width)), u = *(const float4 *)(a + (act ? width : 0));
-      o[0] = __fmul_rn(activate(g.x, 5), u.x);
-      o[1] = __fmul_rn(activate(g.y, 5), u.y);
-      o[2] = __fmul_rn(activate(g.z, 5), u.z);
-      o[3] = __fmul_rn(activate(g.w, 5), u.w);
-    } else {
-      const float4 xv = ((const float4 *)x)[q];
-      const float xi[4] = {xv.x, xv.y, xv.z, xv.w};
-      const float4 bv = MODE == 10 ? ((const float4 *)b)[q] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      const float bi[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t i = i0 + e;
-        if (MODE == 3) {
-          o[e] = __fadd_rn(xi[e], w[i % other_count]);
-        } else if (MODE == 4) {
-          o[e] = __fmul_rn(xi[e], w[i % other_count]);
-        } else if (MODE == 5 || MODE == 6 || MODE == 7) {
-          o[e] = activate(xi[e], MODE == 5 ? 4 : MODE == 6 ? 1 : 2);
-        } else {  // 10
-          const int64_t channel = i % width, batch = i / ((int64_t)width * spatial);
-          const int64_t pb = other_count == width ? 0 : batch;
-          o[e] = __fadd_rn(__fmul_rn(xi[e], w[pb * width + channel]), bi[e]);
-        }
-      }
-    }
-    ((float4 *)y)[q] = make_float4(o[0], o[1], o[2], o[3]);
+                                                                const float *__restrict__ b, uint32_t count4,
+                                                                int width, ElementIndex at, int act) {
+  const uint32_t q = blockIdx.x * kAuxThreads + threadIdx.x;
+  if (q >= count4) return;
+  constexpr bool kOperand = MODE == 3 || MODE == 4 || MODE == 10;
+  const float *a = MODE == 12 ? x + at.operand<MODE>(4u * q) : x;
+  const float4 xv = MODE == 12 ? *(const float4 *)(a + (act ? 0 : width)) : ((const float4 *)x)[q];
+  const float4 bv = MODE == 10 ? ((const float4 *)b)[q] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4 wv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (MODE == 12) {
+    wv = *(const float4 *)(a + (act ? width : 0));
+  } else if (kOperand && QUAD) {
+    wv = *(const float4 *)(w + at.operand<MODE>(4u * q));
+  } else if (kOperand) {
+    wv = make_float4(w[at.operand<MODE>(4u * q)], w[at.operand<MODE>(4u * q + 1u)], w[at.operand<MODE>(4u * q + 2u)],
+                     w[at.operand<MODE>(4u * q + 3u)]);
   }
+  const float xi[4] = {xv.x, xv.y, xv.z, xv.w}, wi[4] = {wv.x, wv.y, wv.z, wv.w}, bi[4] = {bv.x, bv.y, bv.z, bv.w};
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (MODE == 3) o[e] = __fadd_rn(xi[e], wi[e]);
+    else if (MODE == 4) o[e] = __fmul_rn(xi[e], wi[e]);
+    else if (MODE == 10) o[e] = __fadd_rn(__fmul_rn(xi[e], wi[e]), bi[e]);
+    else if (MODE == 12) o[e] = __fmul_rn(activate(xi[e], 5), wi[e]);
+    else o[e] = activate(xi[e], MODE == 5 ? 4 : MODE == 6 ? 1 : 2);
+  }
+  ((float4 *)y)[q] = make_float4(o[0], o[1], o[2], o[3]);
 }
 
 // Mode 8: x[batch][width][spatial] -> y[batch][spatial][width], 32 x 32 tiles through LDS.
@@ -631,6 +659,43 @@ __global__ __launch_bounds__(kAuxThreads) void aux_transpose(float *__restrict__
   __syncthreads();
   for (int c = ty; c < 32; c += 8)
     if (c0 + c < spatial && r0 + tx < width) yb[(size_t)(c0 + c) * width + r0 + tx] = tile[tx][c];
+}
+
+// The same with 64 x 64 tiles and 16-byte loads and stores (width and spatial
+// multiples of 4, x and y 16-byte aligned): four loads in flight per thread,
+// rows of 256 bytes on either side.  Rows of 65 words: the four words of a
+// quad and the 16 quads of a row or column fall into different banks.  us, 32
+// x 32 tiles of single values -> this: 4352 x 6144 58.8 -> 42.1 (5.1 TB/s),
+// 4096 x 3072 30.0 -> 21.2, 4352 x 1536 16.9 -> 11.8, 333 x 1280 4.2 either way.
+__global__ __launch_bounds__(kAuxThreads) void aux_transpose4(float *__restrict__ y, const float *__restrict__ x,
+                                                              int width, int spatial) {
+  __shared__ float tile[64][65];
+  const int batch = blockIdx.z, r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  const float *xb = x + (size_t)batch * width * spatial;
+  float *yb = y + (size_t)batch * width * spatial;
+  const int t4 = 4 * (threadIdx.x & 15), row = threadIdx.x >> 4;  // 16 quads x 16 rows
+  float4 v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int r = min(r0 + row + 16 * u, width - 1), c = min(c0 + t4, spatial - 4);
+    v[u] = *(const float4 *)(xb + (size_t)r * spatial + c);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    float *d = &tile[row + 16 * u][t4];
+    d[0] = v[u].x;
+    d[1] = v[u].y;
+    d[2] = v[u].z;
+    d[3] = v[u].w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int c = row + 16 * u;
+    if (c0 + c < spatial && r0 + t4 < width)
+      *(float4 *)(yb + (size_t)(c0 + c) * width + r0 + t4) =
+          make_float4(tile[t4][c], tile[t4 + 1][c], tile[t4 + 2][c], tile[t4 + 3][c]);
+  }
 }
 
 // Mode 11: one workgroup per (batch, token); threads over heads x pairs.
@@ -650,6 +715,28 @@ __global__ __launch_bounds__(kAuxThreads) void aux_rope(float *__restrict__ y, c
     ys[0] = __fadd_rn(__fmul_rn(x0, m[0]), __fmul_rn(x1, m[1]));
     ys[1] = __fadd_rn(__fmul_rn(x1, m[3]), __fmul_rn(x0, m[2]));
   }
+}
+
+// The same, two pairs (16 bytes) per thread over all quads of x in order (dim
+// % 4 == 0, all operands 16-byte aligned, below 2^31 values): full waves
+// whatever the number of heads.  us, a workgroup per token -> this: 4352 x 6144
+// 46.7 -> 38.5 (5.6 TB/s), 4096 x 3072 22.1 -> 19.9, 4352 x 1536 13.1 -> 11.8.
+__global__ __launch_bounds__(kAuxThreads) void aux_rope4(float *__restrict__ y, const float *__restrict__ x,
+                                                         const float *__restrict__ pe, uint32_t count4, int heads,
+                                                         int tokens, int groups, IndexDivisor by_dim4,
+                                                         IndexDivisor by_heads, IndexDivisor by_tokens) {
+  const uint32_t q = blockIdx.x * kAuxThreads + threadIdx.x, dim4 = by_dim4.d;
+  if (q >= count4) return;
+  const uint32_t row = by_dim4.quotient(q), p = q - row * dim4;  // (batch, token, head), quad
+  const uint32_t task = by_heads.quotient(row), head = row - task * (uint32_t)heads;
+  const uint32_t batch = by_tokens.quotient(task), token = task - batch * (uint32_t)tokens;
+  const float4 *m = (const float4 *)pe + ((size_t)(groups == 1 ? token : task) * dim4 + p) * 2;
+  const float4 v = ((const float4 *)x)[q], a = m[0], c = m[1];
+  ((float4 *)y)[(((size_t)batch * heads + head) * tokens + token) * dim4 + p] =
+      make_float4(__fadd_rn(__fmul_rn(v.x, a.x), __fmul_rn(v.y, a.y)),
+                  __fadd_rn(__fmul_rn(v.y, a.w), __fmul_rn(v.x, a.z)),
+                  __fadd_rn(__fmul_rn(v.z, c.x), __fmul_rn(v.w, c.y)),
+                  __fadd_rn(__fmul_rn(v.w, c.w), __fmul_rn(v.z, c.z)));
 }
 
 // Mode 13: output row r = [attention row r (groups values) | SiLU(gate) * up (width values)].
@@ -782,15 +869,24 @@ int elementwise_grid(int64_t count) {
 template <int MODE>
 void launch_elementwise(float *y, const float *x, const float *w, const float *b, int count, int width, int channels,
                         int spatial, int other_count, int act, hipStream_t st) {
+  constexpr bool kPeriod = MODE == 3 || MODE == 4;
+  const ElementIndex at{index_divisor(kPeriod ? other_count : width), index_divisor((int64_t)width * spatial),
+                        (uint32_t)channels, other_count == width};
   bool vec = count % 4 == 0 && aligned16(x) && aligned16(y) && (MODE != 10 || aligned16(b));
   if (MODE == 12) vec = vec && width % 4 == 0 && channels % 4 == 0;
   if (vec) {
-    const int64_t count4 = count / 4;
-    hipLaunchKernelGGL(aux_elementwise4<MODE>, dim3(elementwise_grid(count4)), dim3(kAuxThreads), 0, st, y, x, w, b,
-                       count4, width, channels, spatial, other_count, act);
+    const int count4 = count / 4;
+    const dim3 grid((count4 + kAuxThreads - 1) / kAuxThreads);
+    const bool quad = kPeriod ? other_count % 4 == 0 && aligned16(w) : MODE != 10 || (width % 4 == 0 && aligned16(w));
+    if (quad)
+      hipLaunchKernelGGL((aux_elementwise4<MODE, true>), grid, dim3(kAuxThreads), 0, st, y, x, w, b, (uint32_t)count4,
+                         width, at, act);
+    else
+      hipLaunchKernelGGL((aux_elementwise4<MODE, false>), grid, dim3(kAuxThreads), 0, st, y, x, w, b,
+                         (uint32_t)count4, width, at, act);
   } else {
     hipLaunchKernelGGL(aux_elementwise<MODE>, dim3(elementwise_grid(count)), dim3(kAuxThreads), 0, st, y, x, w, b,
-                       (int64_t)count, width, channels, spatial, other_count, act);
+                       (int64_t)count, width, at, act);
   }
 }
 
@@ -897,6 +993,11 @@ extern "C" int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, c
       break;
     case 8: {
       if ((int64_t)width * spatial * batch != count) return hb_invalid("hb_model_aux transpose shape");
+      if (width % 4 == 0 && spatial % 4 == 0 && aligned16(d_x) && aligned16(d_y)) {
+        const dim3 grid4((spatial + 63) / 64, (width + 63) / 64, batch);
+        hipLaunchKernelGGL(aux_transpose4, grid4, block, 0, st, d_y, d_x, width, spatial);
+        break;
+      }
       const dim3 grid((spatial + 31) / 32, (width + 31) / 32, batch);
       hipLaunchKernelGGL(aux_transpose, grid, block, 0, st, d_y, d_x, width, spatial);
       break;
@@ -905,11 +1006,21 @@ extern "C" int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, c
       if (!d_w || !d_b) return hb_invalid("hb_model_aux mode 10 parameters");
       launch_elementwise<10>(d_y, d_x, d_w, d_b, count, width, channels, spatial, other_count, activation, st);
       break;
-    case 11:
+    case 11: {
       if (!d_w || width % 2 || (groups != 1 && groups != batch)) return hb_invalid("hb_model_aux rope");
+      const int64_t values = (int64_t)spatial * batch * channels * width;
+      if (width % 4 == 0 && aligned16(d_x) && aligned16(d_y) && aligned16(d_w) && values <= INT32_MAX) {
+        const int64_t count4 = values / 4;
+        const IndexDivisor dim4 = index_divisor(width / 4), heads = index_divisor(channels),
+                           tokens = index_divisor(spatial);
+        hipLaunchKernelGGL(aux_rope4, dim3((uint32_t)((count4 + kAuxThreads - 1) / kAuxThreads)), block, 0, st, d_y, d_x,
+                           d_w, (uint32_t)count4, channels, spatial, groups, dim4, heads, tokens);
+        break;
+      }
       hipLaunchKernelGGL(aux_rope, dim3(spatial * batch), block, 0, st, d_y, d_x, d_w, width, channels, spatial,
                          groups);
       break;
+    }
     case 12:
       if (channels < 2 * width) return hb_invalid("hb_model_aux gated width");
       launch_elementwise<12>(d_y, d_x, d_w, d_b, count, width, channels, spatial, other_count, activation, st);

@@ -502,6 +502,51 @@ def test_aux_gated_gpu(hip, orc, act, rows, width, channels):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("other", [1, 2, 3, 4, 63, 64, 65, 4095, 4096, 4097, 1 << 20, 5000000])
+def test_aux_index_divisors_gpu(hip, orc, other):
+    """Whole and split quads of w, divisors around powers of two, the last quad; bit-exact."""
+    for count in (1 << 20, (1 << 20) + 3):
+        x, w = rng_normal(count, 210), rng_normal(other, 211)
+        kw = dict(mode=3, count=count, width=other, other_count=other)
+        got, _ = run_aux(hip, x, w, None, **kw)
+        assert np.array_equal(got, orc.model_aux(x, w, None, **kw))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,spatial,width", [(3, 4, 37), (2, 77, 100), (1, 1, 4), (5, 8, 1)])
+@pytest.mark.parametrize("per_batch", [False, True])
+def test_aux_modulation_gate_rows_gpu(hip, orc, batch, spatial, width, per_batch):
+    """Rows that quads straddle and rows of whole quads; with and without a remainder."""
+    x = rng_normal(batch * spatial * width, 510)
+    other = width * batch if per_batch else width
+    w, b = rng_normal(other, 511), rng_normal(x.size, 512)
+    kw = dict(mode=10, count=x.size, width=width, spatial=spatial, batch=batch, other_count=other)
+    got, _ = run_aux(hip, x, w, b, **kw)
+    assert np.array_equal(got, orc.model_aux(x, w, b, **kw))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,width,spatial", [(1, 4, 4), (2, 64, 68), (1, 60, 132), (3, 192, 4), (1, 68, 66)])
+def test_aux_transpose_tiles_gpu(hip, orc, batch, width, spatial):
+    x = rng_normal(batch * width * spatial, 410)
+    kw = dict(mode=8, count=x.size, width=width, spatial=spatial, batch=batch)
+    got, _ = run_aux(hip, x, None, None, **kw)
+    assert np.array_equal(got, orc.model_aux(x, None, None, **kw))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,tokens,heads,dim,groups", [(3, 33, 5, 12, 3), (3, 33, 5, 12, 1), (1, 1, 1, 4, 1),
+                                                           (2, 65, 30, 64, 2), (2, 7, 3, 6, 2)])
+def test_aux_rope_quads_gpu(hip, orc, batch, tokens, heads, dim, groups):
+    x = rng_normal(batch * tokens * heads * dim, 610)
+    pe = rope_matrices(groups, tokens, dim, 611)
+    kw = dict(mode=11, count=x.size, width=dim, channels=heads, spatial=tokens, groups=groups, batch=batch,
+              other_count=2 * dim * tokens * groups)
+    got, _ = run_aux(hip, x, pe, None, **kw)
+    assert np.array_equal(got, orc.model_aux(x, pe, None, **kw))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("device", [False, True])
 def test_aux_opcode19_gpu(hip, orc, device):
     """The full opcode through execute_op_simple, host-resident and HBM-resident
