@@ -686,6 +686,42 @@ __global__ __launch_bounds__(64 * WM *WN) void f16_gemm_ring(float *__restrict__
   }
 }
 
+// A workgroup's raw sums into slice blockIdx.y of the workspace, [mp][n] or
+// [n][mp] (channel_major).
+template <int FM, int FN>
+__device__ inline void splitk_store(hb_f32x4 (&acc)[FM][FN], float *__restrict__ ws, int m, int n, int row0, int col0,
+                                    int lane, int channel_major) {
+  // lane l holds rows 4*(l/16)..+3 and column l%16 of each 16x16 block
+  const int mp = (m + 15) / 16 * 16;
+  if (channel_major) {
+    // slice s as [n][mp]: the lane's 4 rows of a column are one 16-byte store
+    float *slice = ws + (size_t)blockIdx.y * mp * n;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int col = col0 + j * 16 + (lane & 15);
+        const int r0 = row0 + i * 16 + 4 * (lane >> 4);
+        if (col < n && r0 < mp) *(hb_f32x4 *)(slice + (size_t)col * mp + r0) = acc[i][j];
+      }
+    return;
+  }
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(ws + (size_t)blockIdx.y * mp * n, 0, (uint32_t)m * (uint32_t)n * 4u, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int col = col0 + j * 16 + (lane & 15);
+      if (col >= n) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = row0 + i * 16 + 4 * (lane >> 4) + r;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r]), rs, (uint32_t)(row * n + col) * 4u, 0, 0);
+      }
+    }
+}
+
 // Split-K form of the ring kernel for up to 128 rows: grid (tiles, splits),
 // split s multiplies k-steps [s*kps, s*kps + kps) of its BM x BN tile (the
 // k loop of f16_gemm_ring on that range) and stores the raw fp32 sums to
@@ -711,35 +747,88 @@ __global__ __launch_bounds__(64 * WM *WN) void f16_ring_splitk(float *__restrict
   const int kt0 = blockIdx.y * kps, kt_n = min(kps, k / 32 - kt0);
   hb_f32x4 acc[FM][FN];
   ring_mainloop<BM, BN, WM, WN, S>(acc, lds, aimg, wpack, m, k, n, m0, n0, wave, lane, kt0, kt_n);
-  // lane l holds rows 4*(l/16)..+3 and column l%16 of each 16x16 block
-  const int mp = (m + 15) / 16 * 16;
-  if (channel_major) {
-    // slice s as [n][mp]: the lane's 4 rows of a column are one 16-byte store
-    float *slice = ws + (size_t)blockIdx.y * mp * n;
+  splitk_store(acc, ws, m, n, m0 + wm * WTM, n0 + wn * WTN, lane, channel_major);
+}
+
+// The same split-K product from the fp32 rows themselves, without the image
+// pass and its launch: a stage holds 128 rows x 32 fp32 values, brought by
+// whole 128-byte lines (a wave's load takes 8 rows; row r's piece p sits in
+// slot (8p + r) ^ 8h of its 1 KB block, h the half of the 16-row block, so that
+// the fragment reads fall into different banks), and 8 KB of weights; the
+// fragments are rounded to fp16 as they are read, as f16_pack_a rounds them,
+// and multiplied in the same order, so the sums have the same bits.  Rows past
+// m repeat the last one (their sums are never read).  Bound by the operand
+// rate into a CU (24 KB per k-step); 8 waves of 32 x 64 with three stages: 4
+// waves of 64 x 64 took 27.6 us and six stages 27.4 where this takes 26.7
+// (1024x5760x640).
+template <int WM, int WN, int S>
+__global__ __launch_bounds__(64 * WM *WN) void f16_rows_splitk(float *__restrict__ ws, const float *__restrict__ x,
+                                                               const int8_t *__restrict__ wpack, int m, int k, int n,
+                                                               int kps, int channel_major) {
+  constexpr int BM = 128, BN = 128, NW = WM * WN;
+  constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
+  constexpr int AB = BM / 16 * 2, NB = AB + BN / 16, PW = NB / NW, PA = AB / NW;  // 1 KB blocks of a stage
+  constexpr int STAGE = NB * kFragBytes;
+  static_assert(AB % NW == 0 && NB % NW == 0, "every wave issues the same loads of either operand");
+  __shared__ __attribute__((aligned(1024))) int8_t lds[S * STAGE];
+  const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
+  int tm, tn;
+  tile_coords_2d<2 * BM, BN>(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm = wave / WN, wn = wave % WN;
+  const int kt_count = k / 32, nblocks = n / 16, kt0 = blockIdx.y * kps, steps = min(kps, kt_count - kt0);
+  const int8_t *src[PW];
+  int stride[PW];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int col = n0 + wn * WTN + j * 16 + (lane & 15);
-        const int r0 = m0 + wm * WTM + i * 16 + 4 * (lane >> 4);
-        if (col < n && r0 < mp) *(hb_f32x4 *)(slice + (size_t)col * mp + r0) = acc[i][j];
-      }
-    return;
+  for (int i = 0; i < PW; ++i) {
+    const int b = i * NW + wave;
+    if (i < PA) {
+      // 8 rows of 128 bytes: row v % 8, piece v / 8 by lane v ^ 8 * (b % 2)
+      const int v = lane ^ (8 * (b & 1));
+      src[i] = (const int8_t *)(x + (size_t)min(m0 + 8 * b + (v & 7), m - 1) * k + 4 * (v >> 3));
+      stride[i] = 128;
+    } else {
+      src[i] = wpack + (size_t)min(n0 / 16 + b - AB, nblocks - 1) * kt_count * kFragBytes + lane * 16;
+      stride[i] = kFragBytes;
+    }
   }
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc(ws + (size_t)blockIdx.y * mp * n, 0, (uint32_t)m * (uint32_t)n * 4u, 0x00020000);
+  // where lane l (row l % 16, values 8 * (l / 16) .. + 7) finds its two pieces
+  const int ar = lane & 15, ap = 2 * (lane >> 4);
+  const int a_lo = ((ar >> 3) * 64 + ((8 * ap + (ar & 7)) ^ (8 * (ar >> 3)))) * 16;
+  const int a_hi = ((ar >> 3) * 64 + ((8 * (ap + 1) + (ar & 7)) ^ (8 * (ar >> 3)))) * 16;
+  hb_f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int col = n0 + wn * WTN + j * 16 + (lane & 15);
-      if (col >= n) continue;
+    for (int j = 0; j < FN; ++j) acc[i][j] = hb_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm * WTM + i * 16 + 4 * (lane >> 4) + r;
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r]), rs, (uint32_t)(row * n + col) * 4u, 0, 0);
-      }
+  for (int s = 0; s < S - 1; ++s)
+    if (s < steps) dma_stage<PW, NW, NB>(lds + s * STAGE, src, stride, kt0 + s, wave, lane);
+  int rd = 0, wr = S - 1;
+  for (int kt = 0; kt < steps; ++kt) {
+    wait_stage<PW, S - 2>(steps - 1 - kt);
+    block_barrier();
+    if (kt + S - 1 < steps)
+      dma_stage<PW, NW, NB>(lds + wr * STAGE, src, stride, kt0 + kt + S - 1, wave, lane);
+    const int8_t *base = lds + rd * STAGE, *la = base + wm * FM * 2 * kFragBytes;
+    const int8_t *lb = base + (AB + wn * FN) * kFragBytes + lane * 16;
+    if (++rd == S) rd = 0;
+    if (++wr == S) wr = 0;
+    hb_f16x8 bf[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) bf[j] = *(const hb_f16x8 *)(lb + j * kFragBytes);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const hb_f32x4 lo = *(const hb_f32x4 *)(la + i * 2 * kFragBytes + a_lo);
+      const hb_f32x4 hi = *(const hb_f32x4 *)(la + i * 2 * kFragBytes + a_hi);
+      const hb_f16x8 af = {(_Float16)lo[0], (_Float16)lo[1], (_Float16)lo[2], (_Float16)lo[3],
+                           (_Float16)hi[0], (_Float16)hi[1], (_Float16)hi[2], (_Float16)hi[3]};
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[j], acc[i][j], 0, 0, 0);
     }
+  }
+  splitk_store(acc, ws, m, n, m0 + wm * FM * 16, n0 + wn * FN * 16, lane, channel_major);
 }
 
 // ---------------------------------------------------------------------------
@@ -2312,11 +2401,11 @@ int launch_ring(float *y, const float *x, const uint16_t *packed, const float *b
   return hb_check_launch("f16_gemm_ring");
 }
 
-// Split-K ring path for m <= 256: fp16 activation image, f16_ring_splitk on
-// 128 x 128 tiles with K split so that the launch has about two workgroups
-// per CU (at most kMaxRingSplits slices), then f16_skinny_epilogue.  It
+// Split-K ring path: 128 x 128 tiles with K split (at most kMaxRingSplits
+// slices) by f16_rows_splitk on the fp32 rows or by f16_ring_splitk on their
+// fp16 image, then f16_skinny_epilogue.  Up to 256 rows it
 // replaces the few-rows split-K kernel from 33 rows on, whose every column
-// group re-reads the fp32 rows (measured, us, few-rows / this path:
+// group re-reads the fp32 rows (measured, us, few-rows / the image form:
 // 77x10240x4096 60.7 / 25.0, 128x10240x4096 120 / 31, 77x4096x4096 25.4 /
 // 16.6, 64x4096x4096 19.3 / 16.0, 48x2048x8192 20.4 / 17.0, 77x1280x5120
 // 17.1 / 14.3; at 32 rows and fewer the few-rows kernel stays ahead:
@@ -2328,52 +2417,94 @@ int launch_ring(float *y, const float *x, const uint16_t *packed, const float *b
 // (256x4096x4096 27.7 -> 28.4).
 constexpr int kMaxRingSplits = 8;
 
+long long tiles128(int m, int n) { return (long long)((m + 127) / 128) * ((n + 127) / 128); }
+
+// Up to 256 rows about two workgroups per CU.  From 257 rows one per CU where
+// that gives three slices or more, else two: every slice is written and read
+// again, and a launch of one and a half workgroups per CU takes as long as two
+// (packed image, us, two per CU rounded up -> this: 1024x5760x640 33.5 -> 29.1,
+// 512x11520x1280 45.1 -> 39.3, 700x8640x1280 43.1 -> 39.0, 1500x4608x960 45.7
+// -> 39.4, 1024x11520x1280 71.7 -> 61.1).
 int ring_splits(int m, int k, int n) {
-  const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
-  const long long want = (2LL * compute_units() + tiles - 1) / tiles;
+  const long long tiles = tiles128(m, n), cus = compute_units();
+  long long want = (2 * cus + tiles - 1) / tiles;
+  if (m > 256) want = cus / tiles >= 3 ? cus / tiles : 2 * cus / tiles;
   const int kblocks = k / 32;
   int splits = (int)std::min<long long>(std::min<long long>(want, kMaxRingSplits), kblocks);
   return splits < 1 ? 1 : splits;
 }
 
-// 257 to kRingSplitRows rows and k >= 2048: the split-K ring path where
-// 128 x 128 tiles fill at most half of the CUs (the few-tile, long-k
-// products of im2col convolutions).  Measured, us, ring kernel -> split-K,
-// mode 0: 512x11520x1280 71.3 -> 43.5, 1024x11520x1280 84.5 -> 73.5,
-// 1024x4608x512 34.8 -> 25.2, 1024x5760x640 41.3 -> 31.5, 512x5760x1280
-// 38.0 -> 28.3, 2048x4608x512 39.9 -> 38.2, 1024x2880x640 23.4 -> 23.0; at
-// 160 tiles (2048x11520x1280) 122.5 against 120.3.
-constexpr int kRingSplitRows = 2048;
-
-bool wide_splitk_shape(int m, int k, int n) {
-  const long long tiles128 = ((m + 127) / 128) * (long long)((n + 127) / 128);
-  return m > 256 && m <= kRingSplitRows && k >= 2048 && 2 * tiles128 <= compute_units();
+// Slices that hold k-steps, of kps k-steps each (the last may hold fewer).
+int ring_slices(int m, int k, int n, int &kps) {
+  const int splits = ring_splits(m, k, n);
+  kps = (k / 32 + splits - 1) / splits;
+  return (k / 32 + kps - 1) / kps;
 }
 
-// Workspace of the split-K ring path: the fp16 image and the slices; 0 where
-// the path does not run (more than 256 rows outside wide_splitk_shape).
+// Whether the split-K path multiplies the fp32 rows themselves
+// (f16_rows_splitk) or an fp16 image of them: at most one workgroup per CU (a
+// second one has to share the CU's operand rate, of which fp32 rows take
+// half more), and the k-steps' extra time (0.14 us each) below what the image
+// pass takes (3.9 us and 0.12 per MB of x).  Measured, us, image / rows, same
+// slices: 1024x5760x640 (30 k-steps a slice) 29.1 / 26.7, 2048x4608x512 (36)
+// 34.8 / 29.0, 2048x2880x640 (30) 29.6 / 27.6, 2048x11520x256 (45) 53.0 / 34.5,
+// 400x2304x512 (9) 16.7 / 13.9, 77x4096x4096 (16) 17.2 / 14.9, 100x3072x3072
+// (12) 17.0 / 14.6; left on the image: 512x11520x1280 (60) 39.3 / 41.1,
+// 128x10240x4096 (40) 27.9 / 30.8, 700x8640x1280 (68) 39.0 / 44.2.
+bool splitk_rows(int m, int k, int n) {
+  int kps = 0;
+  const int slices = ring_slices(m, k, n, kps);
+  return tiles128(m, n) * slices <= compute_units() && kps <= 28.0 + 0.85e-6 * 4.0 * m * (double)k;
+}
+
+// From 257 rows and k >= 2048: the split-K ring path where 128 x 128 tiles
+// fill at most half of the CUs, and above kRingSplitRows rows where they fill
+// at most a third (the few-tile, long-k products of im2col convolutions).
+// From kUnsplitRows rows the sums stay unsplit: there the ring and the
+// activation-streaming kernel give the same bits, whichever takes the shape.
+// Measured, us, mode 3, ring kernel -> split-K: 512x11520x1280 71.3 -> 39.3,
+// 1024x11520x1280 84.5 -> 61.1, 1024x4608x512 34.8 -> 18.8, 1024x5760x640 41.3
+// -> 26.7, 2048x4608x512 39.9 -> 29.0, 2048x2880x640 41.2 -> 27.6, 3000x2304x256
+// 30.0 -> 19.7, 3000x4608x320 45.2 -> 34.5,
+// 2500x8640x384 72.6 -> 44.3; at 160 tiles (2048x11520x1280) 122.5 against
+// 120.3, and with shorter sums the ring stays ahead (1000x1152x640 14.4 / 16.8,
+// 512x1536x1536 15.7 / 18.4).
+constexpr int kRingSplitRows = 2048, kUnsplitRows = 4096;
+
+bool wide_splitk_shape(int m, int k, int n) {
+  if (m <= 256 || m >= kUnsplitRows || k < 2048) return false;
+  return tiles128(m, n) * (m <= kRingSplitRows ? 2 : 3) <= compute_units();
+}
+
+// Workspace of the split-K ring path: the fp16 image (none from 257 rows where
+// the fp32 rows are multiplied) and the slices; 0 where the path does not run
+// (more than 256 rows outside wide_splitk_shape).
 size_t ring_splitk_bytes(int m, int k, int n) {
   if (m < 1 || k < 32 || n < 32 || (m > 256 && !wide_splitk_shape(m, k, n))) return 0;
   const int slices = m <= 256 ? kMaxRingSplits : ring_splits(m, k, n);
-  return a_image_bytes(m, k) + (size_t)slices * (size_t)((m + 15) / 16 * 16) * (size_t)n * 4u;
+  const size_t image = m > 256 && splitk_rows(m, k, n) ? 0 : a_image_bytes(m, k);
+  return image + (size_t)slices * (size_t)((m + 15) / 16 * 16) * (size_t)n * 4u;
 }
 
 int launch_ring_splitk(float *y, const float *x, const uint16_t *packed, const float *bias, int m, int k, int n,
                        int channels, int mode, void *ws, hipStream_t st) {
-  const int mp = (m + 15) / 16 * 16;
-  const size_t slots = (size_t)mp * k / 8u;
-  const int pg = (int)((slots + 255) / 256 < 65536 ? (slots + 255) / 256 : 65536);
-  hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)ws, x, m, k, mp);
-  int rc = hb_check_launch("f16_pack_a");
-  if (rc) return rc;
-  const int splits = ring_splits(m, k, n);
-  const int kps = (k / 32 + splits - 1) / splits;
-  const int used = (k / 32 + kps - 1) / kps;  // slices that hold k-steps
-  float *part = (float *)((uint8_t *)ws + a_image_bytes(m, k));
-  const int tiles = ((m + 127) / 128) * ((n + 127) / 128);
-  const int cm = mode == 3;
-  hipLaunchKernelGGL((f16_ring_splitk<128, 128, 2, 2, 4>), dim3(tiles, used), dim3(256), 0, st, part,
-                     (const int8_t *)ws, (const int8_t *)packed, m, k, n, kps, cm);
+  const int mp = (m + 15) / 16 * 16, cm = mode == 3;
+  int kps = 0, rc = 0;
+  const int used = ring_slices(m, k, n, kps);
+  const dim3 grid((int)tiles128(m, n), used);
+  const int8_t *w = (const int8_t *)packed;
+  float *part = (float *)ws;
+  if (splitk_rows(m, k, n)) {
+    hipLaunchKernelGGL((f16_rows_splitk<4, 2, 3>), grid, dim3(512), 0, st, part, x, w, m, k, n, kps, cm);
+  } else {
+    const size_t slots = (size_t)mp * k / 8u;
+    const int pg = (int)((slots + 255) / 256 < 65536 ? (slots + 255) / 256 : 65536);
+    hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)ws, x, m, k, mp);
+    if ((rc = hb_check_launch("f16_pack_a"))) return rc;
+    part = (float *)((uint8_t *)ws + a_image_bytes(m, k));
+    hipLaunchKernelGGL((f16_ring_splitk<128, 128, 2, 2, 4>), grid, dim3(256), 0, st, part, (const int8_t *)ws, w, m, k,
+                       n, kps, cm);
+  }
   rc = hb_check_launch("f16_ring_splitk");
   if (rc) return rc;
   if (cm) {

@@ -247,9 +247,10 @@ int hb_f16_gemm(float *d_y, const float *d_x, const uint16_t *d_packed, const fl
 
 /* Workspace of hb_f16_gemm_ws: the largest of the few-rows (m <= 128) split-K
  * partial sums, for 64 or more rows and at least 4 GFLOP the fp16 activation
- * image of the ring path (2 * ceil(m/16)*16 * k bytes), and for m <= 128 that
- * image plus eight fp32 partial-sum slices of ceil(m/16)*16 x n for m <= 256
- * (the split-K ring path); 0 when none applies (the tiled kernel needs none). */
+ * image of the ring path (2 * ceil(m/16)*16 * k bytes), and for the split-K
+ * ring path its fp32 partial-sum slices of ceil(m/16)*16 x n, at most eight,
+ * with that image for m <= 256 and wherever the image is what it multiplies;
+ * 0 when none applies (the tiled kernel needs none). */
 size_t hb_f16_workspace_bytes(int m, int k, int n);
 
 /* Tuning and test hook of the F16 path for 64 rows or more with a workspace:
@@ -280,8 +281,8 @@ int hb_f16_force_wide(int setting);
  * HTP_OPS_AMD_F16_XSTREAM gives the initial value. */
 int hb_f16_force_xstream(int setting);
 
-/* Pins the split-K ring path of hb_f16_gemm_ws (f16_ring_splitk slices added
- * in order by a readout kernel): -1 restores the automatic choice, 0 never
+/* Pins the split-K ring path of hb_f16_gemm_ws (slices of f16_rows_splitk
+ * or f16_ring_splitk added in order by a readout kernel): -1 restores the automatic choice, 0 never
  * (the ring or tiled kernel, whose sums are those of hb_f16_gemm), 1 for
  * every m <= 256 given a large enough workspace (from 257 rows it runs only
  * where the automatic choice takes it).  Returns the previous
@@ -295,10 +296,11 @@ int hb_f16_force_splitk(int setting);
  * (of the size hb_f16_gemm would use) number no more than the device's CUs, K
  * is split across workgroups and the partial sums are added in a fixed order
  * before the fp16 readout rounding and the epilogue (two kernels; from 33
- * rows on, x is first converted to fp16 MFMA tiles and each split covers all
- * rows of a 128 x 128 tile, so the weights are read once).  The same
+ * rows on, each split covers 128 x 128 tiles, and x is converted to fp16 as it
+ * is read, or before in a third kernel where many tiles read it).  The same
  * split-K ring path serves 257 to 2048 rows with k >= 2048 where 128 x 128
- * output tiles would fill at most half of the CUs.
+ * output tiles would fill at most half of the CUs, and up to 4095 rows where
+ * they would fill at most a third.
  * Otherwise, with a workspace of at least hb_f16_workspace_bytes, a 16-byte
  * aligned output and 64 or more rows (4 GFLOP or more), x is converted once
  * into fp16 MFMA tiles in the workspace and both operands stream through the

@@ -727,6 +727,39 @@ def test_f16_channel_major_matches_row_major(hip, orc, m, k, n, channels, ring):
         np.testing.assert_array_equal(got, yt.read(np.uint32, m * channels).reshape(channels, m))
 
 
+@pytest.mark.parametrize("m,k,n,channels,mode,bias", [
+    (33, 3104, 96, 96, 0, False),      # one row tile, n under a tile, a last slice of fewer k-steps
+    (128, 2048, 3072, 3072, 2, True),  # whole tiles, a few k-steps per slice
+    (129, 4096, 160, 130, 3, True),    # one row past a tile, channels < n, m % 4 != 0
+    (257, 2080, 352, 352, 1, True),    # 65 k-steps, one row past two tiles
+    (2053, 2048, 128, 128, 3, False),  # above 2048 rows, m % 4 != 0
+    (2900, 2048, 288, 288, 0, True),   # above 2048 rows, 69 tiles: three slices
+    (300, 9216, 1216, 1216, 0, True),  # long slices: the fp16 image
+])
+def test_f16_splitk_forms(hip, orc, m, k, n, channels, mode, bias):
+    """Split-K on the fp32 rows and on their fp16 image, within the F16 bound
+    of the oracle, with what a workspace of exactly the asked size holds."""
+    ws = hip.DeviceBuffer(hip.f16_workspace_bytes(m, k, n))
+    x, w, perm, b = f16_case(orc, m, k, n, seed=m + k + n + 3, bias=bias)
+    packed = hip.f16_prepack(hip.DeviceBuffer.from_array(perm), k, n)
+    bvec = None if b is None else b[:channels].copy()
+    bd = hip.DeviceBuffer.from_array(bvec) if bias else None
+    y = hip.DeviceBuffer(m * channels * 4)
+    y.fill(0xFF)
+    hip.f16_gemm(y, hip.DeviceBuffer.from_array(x), packed, bd, m, k, n, channels, mode, workspace=ws)
+    hip.sync()
+    ref = orc.f16_gemm_epilogue(x, perm, bvec, m, k, n, channels, mode)
+    v_ref, absdot = orc.f16_gemm_epilogue(x, perm, None, m, k, n, n, 0), f16_abs_dot(x, w)
+    if mode == 3:
+        got = y.read(np.float32, m * channels).reshape(channels, m)
+        v_ref, absdot = v_ref.T[:channels], absdot.T[:channels]
+        bias_cols = np.abs(bvec)[:, None] if bias else 0.0
+    else:
+        got = y.read(np.float32, m * n).reshape(m, n)
+        bias_cols = np.abs(b)[None, :] if bias else 0.0
+    assert_f16_close(got, ref, v_ref, bias_cols, absdot, k)
+
+
 def test_f16_workspace_covers_only_the_paths_that_run(hip):
     """The workspace holds split-K slices only for shapes that take the
     split-K ring path: many output tiles at 2048 rows need the fp16 image
