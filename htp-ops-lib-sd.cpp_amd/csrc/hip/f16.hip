@@ -2444,17 +2444,20 @@ int ring_slices(int m, int k, int n, int &kps) {
 // Whether the split-K path multiplies the fp32 rows themselves
 // (f16_rows_splitk) or an fp16 image of them: at most one workgroup per CU (a
 // second one has to share the CU's operand rate, of which fp32 rows take
-// half more), and the k-steps' extra time (0.14 us each) below what the image
-// pass takes (3.9 us and 0.12 per MB of x).  Measured, us, image / rows, same
-// slices: 1024x5760x640 (30 k-steps a slice) 29.1 / 26.7, 2048x4608x512 (36)
-// 34.8 / 29.0, 2048x2880x640 (30) 29.6 / 27.6, 2048x11520x256 (45) 53.0 / 34.5,
-// 400x2304x512 (9) 16.7 / 13.9, 77x4096x4096 (16) 17.2 / 14.9, 100x3072x3072
-// (12) 17.0 / 14.6; left on the image: 512x11520x1280 (60) 39.3 / 41.1,
-// 128x10240x4096 (40) 27.9 / 30.8, 700x8640x1280 (68) 39.0 / 44.2.
+// half more), and no more k-steps a slice than the image pass pays for (its
+// launch about 20, its traffic 0.9 per MB of x; the line lies between the
+// pairs below).  Measured, us, image / rows, same slices (k-steps each):
+// 1024x5760x640 (30) 29.1 / 26.7, 2048x4608x512 (36) 34.8 / 29.0, 900x10240x512
+// (40) 35.8 / 30.5, 2048x11520x256 (45) 53.0 / 34.5, 700x5760x640 (23) 25.4 /
+// 22.9, 77x4096x4096 (16) 17.2 / 14.9, 77x5120x3072 (20) 17.0 / 16.0,
+// 250x2048x1024 (8) 16.2 / 12.3; left on the image: 171x6144x1536 (24) 19.4 /
+// 20.8, 171x8192x2048 (32) 23.8 / 26.2, 120x8640x960 (34) 22.5 / 23.8,
+// 500x6144x1536 (39) 27.9 / 30.4, 512x11520x1280 (60) 39.3 / 41.1,
+// 128x10240x4096 (40) 27.9 / 30.8.
 bool splitk_rows(int m, int k, int n) {
   int kps = 0;
   const int slices = ring_slices(m, k, n, kps);
-  return tiles128(m, n) * slices <= compute_units() && kps <= 28.0 + 0.85e-6 * 4.0 * m * (double)k;
+  return tiles128(m, n) * slices <= compute_units() && kps <= 20.0 + 0.9e-6 * 4.0 * m * (double)k;
 }
 
 // From 257 rows and k >= 2048: the split-K ring path where 128 x 128 tiles
