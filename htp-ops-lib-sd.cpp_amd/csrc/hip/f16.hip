@@ -1195,16 +1195,17 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void f16_gemm_square(float *__r
 struct QkvPart {
   const int8_t *aimg, *wpack;
   const float *bias, *q_norm, *k_norm;
-  int m, rope_off, out_tile0;
+  int m, rope_off, rope_rows, out_tile0;  // rope_rows: tokens that are rotated (qkv_rope.h)
 };
 
 template <int HD, int WHICH, int FN>
 __device__ __attribute__((always_inline)) inline void qkv_rows_store(hb_f32x4 (&acc)[2][FN], uint16_t *dst,
                                                                      const QkvPart &part, const float *gamma,
-                                                                     const float *pe, int rope_count, int token_tiles,
-                                                                     int head0, int n0, int row, int lane) {
+                                                                     const float *pe, int token_tiles, int head0,
+                                                                     int n0, int row, int lane) {
   // The rotary matrices (4 floats per column pair) of this lane's rows, read
-  // once for all heads of the tile; a row that is not rotated reads some row's.
+  // once for all heads of the tile; a row that is not rotated (also one past
+  // the part's tokens) reads those of the part's last rotated row.
   constexpr int FH = HD / 16;
   const int rows = min(32, part.m - row);
   const size_t head_words = (size_t)token_tiles * (HD / 32) * 1024;
@@ -1212,10 +1213,11 @@ __device__ __attribute__((always_inline)) inline void qkv_rows_store(hb_f32x4 (&
   for (int i = 0; i < 2; ++i) {
     hb_f32x4 mat[FH][2] = {};
     bool rot = false;
-    if (WHICH < 2 && pe) {
-      const int r = 16 * i + (lane & 15), token = part.rope_off + row + r;
-      rot = r < rows && token < rope_count;
-      const float *pr = pe + ((size_t)min(token, rope_count - 1) * (HD / 2) + 2 * (lane >> 4)) * 4u;
+    if (WHICH < 2 && part.rope_rows > 0) {
+      const int t = row + 16 * i + (lane & 15);
+      rot = t < part.rope_rows;
+      const float *pr =
+          pe + ((size_t)qkv_rope_row(part.rope_off, part.rope_rows, t) * (HD / 2) + 2 * (lane >> 4)) * 4u;
 #pragma unroll
       for (int j = 0; j < FH; ++j)
 #pragma unroll
@@ -1232,7 +1234,7 @@ template <int HD, int BN, int S, int D>
 __global__ __launch_bounds__(64 * kWideWaves, BN == 64 ? 4 : 2) void f16_qkv_rows(uint16_t *__restrict__ q, uint16_t *__restrict__ k,
                                                                   uint16_t *__restrict__ v, QkvPart part0,
                                                                   QkvPart part1, const float *__restrict__ pe,
-                                                                  int rope_count, int kdim, int n_heads,
+                                                                  int kdim, int n_heads,
                                                                   int token_tiles, int bands0, int bands) {
   static_assert(BN % HD == 0, "whole heads per tile");
   constexpr int FM = 2, FN = BN / 16;
@@ -1255,11 +1257,11 @@ __global__ __launch_bounds__(64 * kWideWaves, BN == 64 ? 4 : 2) void f16_qkv_row
   if (row >= part.m) return;
   const int which = n0 / q_cols, head0 = (n0 % q_cols) / HD;
   if (which == 0)
-    qkv_rows_store<HD, 0, FN>(acc, q, part, part.q_norm, pe, rope_count, token_tiles, head0, n0, row, lane);
+    qkv_rows_store<HD, 0, FN>(acc, q, part, part.q_norm, pe, token_tiles, head0, n0, row, lane);
   else if (which == 1)
-    qkv_rows_store<HD, 1, FN>(acc, k, part, part.k_norm, pe, rope_count, token_tiles, head0, n0, row, lane);
+    qkv_rows_store<HD, 1, FN>(acc, k, part, part.k_norm, pe, token_tiles, head0, n0, row, lane);
   else
-    qkv_rows_store<HD, 2, FN>(acc, v, part, nullptr, nullptr, 0, token_tiles, head0, n0, row, lane);
+    qkv_rows_store<HD, 2, FN>(acc, v, part, nullptr, nullptr, token_tiles, head0, n0, row, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2934,8 +2936,10 @@ int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_
     if (!aligned(p.d_x, 16) || !aligned(p.d_packed, 16) || (p.d_bias && !aligned(p.d_bias, 4)))
       return hb_invalid("hb_qkv_gemm alignment");
     if (p.rope_offset < 0 && n_parts > 1) return hb_invalid("hb_qkv_gemm_parts rope offset");
+    // the reference skips the rotation without a table, a count or a valid offset
+    const int rotated = d_pe && p.rope_offset >= 0 ? qkv_rope_rows(p.rope_offset, rope_count, p.tokens) : 0;
     part[i] = {(const int8_t *)d_workspace + need, (const int8_t *)p.d_packed, p.d_bias, p.d_q_norm, p.d_k_norm,
-               p.tokens, p.rope_offset, p.out_offset / 32};
+               p.tokens, p.rope_offset, rotated, p.out_offset / 32};
     bands[i] = (p.tokens + kWideRows - 1) / kWideRows;
     need += a_image_bytes(p.tokens, input_dim);
     slots += (size_t)((p.tokens + 15) / 16 * 16) * (size_t)input_dim / 8u;
@@ -2944,7 +2948,6 @@ int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_
   if (!aligned(d_q, 16) || !aligned(d_k, 16) || !aligned(d_v, 16) || !aligned(d_workspace, 256) ||
       (d_pe && !aligned(d_pe, 16)))
     return hb_invalid("hb_qkv_gemm alignment");
-  if (d_pe && (parts[0].rope_offset < 0 || rope_count <= 0)) d_pe = nullptr;  // the reference skips the rotation
   hipStream_t st = hb_resolve_stream(s);
   const int pg = (int)((slots + 255) / 256 < 65536 ? (slots + 255) / 256 : 65536);
   if (n_parts == 2) {
@@ -2961,13 +2964,13 @@ int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_
   const dim3 grid(all * (n / bn)), block(64 * kWideWaves);
   if (bn == 192)
     hipLaunchKernelGGL((f16_qkv_rows<64, 192, 5, 3>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
-                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+                       input_dim, n_heads, token_tiles, bands[0], all);
   else if (bn == 64)
     hipLaunchKernelGGL((f16_qkv_rows<64, 64, 5, 3>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
-                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+                       input_dim, n_heads, token_tiles, bands[0], all);
   else
     hipLaunchKernelGGL((f16_qkv_rows<128, 128, 6, 4>), grid, block, 0, st, d_q, d_k, d_v, part[0], part[1], d_pe,
-                       rope_count, input_dim, n_heads, token_tiles, bands[0], all);
+                       input_dim, n_heads, token_tiles, bands[0], all);
   return hb_check_launch("f16_qkv_rows");
 }
 

@@ -28,6 +28,8 @@
 
 #include <cstdint>
 
+#include "qkv_rope.h"
+
 namespace {
 
 constexpr int kQkvThreads = 256;  // 4 waves; a wave takes two rows at a time (one per 32 lanes)

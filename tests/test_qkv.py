@@ -17,12 +17,16 @@ GEMM output; the four opcodes through execute_op_simple are bit-exact against
 the oracle post-processing of the library's own F16 GEMM output, and within
 the reference test's 0.03 of its float reference.
 """
+import os
 import struct
+import subprocess
 
 import numpy as np
 import pytest
 
 import htp_ops as h
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 # ---------------------------------------------------------------- helpers ----
 
@@ -449,6 +453,49 @@ def test_qkv_payload_sizes(qbufs):
         assert h.execute(op, b"")[0] == -1, op
 
 
+ROPE_WALK = r"""
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include "qkv_rope.h"
+// offset, count, tokens: rotated tokens, and the highest table row that the
+// lanes of whole 32-token tiles read (-1: none)
+int main(int, char **v) {
+  const int offset = atoi(v[1]), count = atoi(v[2]), tokens = atoi(v[3]);
+  const int n = qkv_rope_rows(offset, count, tokens);
+  long long most = -1;
+  for (int t = 0; n > 0 && t < (tokens + 31) / 32 * 32; ++t) most = std::max<long long>(most, qkv_rope_row(offset, n, t));
+  printf("%d %lld\n", n, most);
+}
+"""
+
+
+def test_rotary_rows_read(tmp_path):
+    """The fused kernels load a rotary matrix for every lane of a 32-token
+    tile: no row past the last rotated token is read, whatever the offsets of
+    a dual request and however many tokens the count allows."""
+    src, exe = tmp_path / "walk.cpp", tmp_path / "walk"
+    src.write_text(ROPE_WALK)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", os.path.join(REPO, "htp-ops-lib-sd.cpp_amd", "csrc", "hip"),
+                    str(src), "-o", str(exe)], check=True)
+
+    def walk(offset, count, tokens):
+        out = subprocess.run([str(exe), str(offset), str(count), str(tokens)], check=True, capture_output=True, text=True)
+        return tuple(map(int, out.stdout.split()))
+
+    for image, text, io, to in ((32, 601, 0, 0), (256, 300, 0, 0), (160, 333, 40, 7), (64, 45, 3, 70), (32, 1, 0, 32)):
+        table, count = max(io + image, to + text), image + text
+        for off, tokens in ((io, image), (to, text)):
+            rotated, most = walk(off, count, tokens)
+            assert rotated == max(0, min(tokens, count - off)) and most == off + rotated - 1
+            assert most < table, (image, text, io, to)
+    top = 2 ** 31 - 1
+    for off, count, tokens in ((0, 1, 33), (5, 5, 64), (9, 3, 64), (top - 5, 10, 64), (top - 5, top, 64), (0, top, 64),
+                               (0, 0, 32), (0, -1, 32)):
+        rotated = max(0, min(tokens, count - off))
+        assert walk(off, count, tokens) == (rotated, off + rotated - 1 if rotated else -1)
+
+
 @pytest.mark.parametrize("heads,hd", [(16, 64), (24, 32), (24, 256), (38, 128), (0, 64), (-24, 64)])
 def test_qkv_unsupported_shapes(qbufs, heads, hd):
     big = qbufs[0]
@@ -786,6 +833,50 @@ def test_hb_qkv_gemm_parts_equal_gemm_then_post(hip, image, text, n_heads, hd, k
             # to about 4 x 1.5 in fp16, whose own rounding adds as much
             fa, fb = (v.view(np.float16).astype(np.float32) for v in (a, b))
             assert np.all(np.abs(fa - fb) <= 2 ** -9 * (1.0 + np.abs(fb))), which
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("image,text,io,to,n_heads,hd", [
+    (256, 300, 0, 0, 24, 64),    # one range of positions: the table ends inside the text part's last row tile
+    (160, 333, 40, 7, 30, 64),   # overlapping ranges, one head per tile
+    (288, 257, 0, 100, 24, 128), # one token in the last row tile
+    (2048, 301, 0, 0, 24, 64),   # three heads per tile
+])
+def test_qkv_dual_rotary_table_of_exactly_the_rows(hip, image, text, io, to, n_heads, hd):
+    """A table of max(image offset + image, text offset + text) rows, which is
+    all a dual request has to bring, where image + text is more: both parts
+    (one launch) equal, bit for bit, their unsplit products post-processed
+    each by itself."""
+    k, count = 64, image + text
+    rng = np.random.default_rng(image + text)
+    cols, tiles = 3 * n_heads * hd, (image + text + 31) // 32
+    size = n_heads * h.qkv_head_elems(tiles, hd)
+    rows = max(io + image, to + text)
+    assert rows < count
+    _, _, _, _, pe = post_inputs(32, 1, hd, 5, rope_tokens=rows)
+    assert pe.size == rows * hd // 2 * 4
+    pe_dev = dev(pe)
+    parts, want, got = [], *[[dev(np.full(size, 0x1234, np.uint16)) for _ in range(3)] for _ in range(2)]
+    prev = h.f16_force_splitk(0)
+    try:
+        for tokens, off, out in ((image, io, 0), (text, to, image)):
+            x = dev(rng.normal(0, 1, (tokens, k)).astype(np.float32))
+            w = h.f16_prepack(dev(h.permute_f16(rng.normal(0, 0.05, (k, cols)).astype(np.float16).view(np.uint16))), k,
+                              cols)
+            qn, kn = (dev(rng.uniform(0.5, 1.5, hd).astype(np.float32)) for _ in range(2))
+            parts.append((x, w, None, qn, kn, off, tokens, out))
+            raw = h.DeviceBuffer(tokens * cols * 4)
+            h.f16_gemm(raw, x, w, None, tokens, k, cols, cols, 0)
+            h.qkv_post(*want, raw, None, qn, kn, pe_dev, off, count, tokens, n_heads, hd, tiles, out)
+            h.sync()
+    finally:
+        h.f16_force_splitk(prev)
+    ws = h.DeviceBuffer(h.qkv_gemm_workspace_bytes(image, k) + h.qkv_gemm_workspace_bytes(text, k))
+    h.qkv_gemm_parts(*got, parts, pe_dev, count, k, n_heads, hd, tiles, ws)
+    h.sync()
+    for which, (g, w) in enumerate(zip(got, want)):
+        a, b = g.read(np.uint16, size), w.read(np.uint16, size)
+        assert np.array_equal(a, b), (which, int((a != b).sum()))
 
 
 @pytest.mark.gpu
