@@ -67,13 +67,14 @@ __device__ inline int block_index(int r, int c) {
 // src: row 0, column 0 of head 0's input (f32, or fp16 holding the same
 // fp16-exact values; rows src_stride elements apart);
 // bias: head 0's first column (NULL: none); rows: valid rows (1..32);
-// token0: the call's token index of row 0 (for the rotary matrices);
+// token0: the call's token index of row 0; tokens below rope_rows (at most the
+// call's tokens) are rotated, token t by row rope_off + t of pe;
 // blk: NH * HD * 32 halfwords of LDS, 16-byte aligned, for the packed blocks;
 // head h's block goes to dst + head_base + h * head_stride.
 template <int HD, int WHICH, int NH, typename T>
 __device__ void qkv_blocks(uint16_t *__restrict__ blk, uint16_t *__restrict__ dst, const T *__restrict__ src,
                            int src_stride, const float *__restrict__ bias, const float *__restrict__ gamma,
-                           const float *__restrict__ pe, int rope_off, int rope_count, int rows, int token0, int tt,
+                           const float *__restrict__ pe, int rope_off, int rope_rows, int rows, int token0, int tt,
                            int token_tiles, size_t head_base, size_t head_stride) {
   constexpr int CH = HD / 64;  // 64-column chunks; lane j holds columns 64d+j and 64d+32+j
   constexpr int E = 2 * CH;    // values per lane and row
@@ -106,12 +107,11 @@ __device__ void qkv_blocks(uint16_t *__restrict__ blk, uint16_t *__restrict__ ds
 #pragma unroll
   for (int i = 0; i < PAIRS; ++i) {
     const int r = 2 * (wave + 4 * i) + half;
-    const int token = rope_off + token0 + r;
-    rot[i] = ROPE_OK && pe && r < rows && token < rope_count;
+    rot[i] = ROPE_OK && token0 + r < rope_rows;
     if (ROPE_OK) {
 #pragma unroll
       for (int e = 0; e < E; ++e)
-        m[i][e] = rot[i] ? *(const float4 *)(pe + ((size_t)token * (HD / 2) + (size_t)(col(e) >> 1)) * 4u)
+        m[i][e] = rot[i] ? *(const float4 *)(pe + ((size_t)(rope_off + token0 + r) * (HD / 2) + (size_t)(col(e) >> 1)) * 4u)
                          : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
@@ -137,7 +137,7 @@ __device__ void qkv_blocks(uint16_t *__restrict__ blk, uint16_t *__restrict__ ds
         const float inv = qkv_rsqrt(__fadd_rn(__fdiv_rn(sum, (float)HD), 1.0e-6f));
 #pragma unroll
         for (int e = 0; e < E; ++e) v[h][i][e] = __fmul_rn(__fmul_rn(v[h][i][e], inv), g[e]);
-        if (pe) {
+        if (rope_rows > 0) {
           // the pair of column c is c ^ 1, held by lane j ^ 1
 #pragma unroll
           for (int e = 0; e < E; ++e) {
@@ -180,9 +180,9 @@ __device__ void qkv_blocks(uint16_t *__restrict__ blk, uint16_t *__restrict__ ds
 template <int HD, int WHICH, typename T>
 __device__ void qkv_block(uint16_t *__restrict__ blk, uint16_t *__restrict__ dst, const T *__restrict__ src,
                           int src_stride, const float *__restrict__ bias, const float *__restrict__ gamma,
-                          const float *__restrict__ pe, int rope_off, int rope_count, int rows, int token0, int tt,
+                          const float *__restrict__ pe, int rope_off, int rope_rows, int rows, int token0, int tt,
                           int token_tiles, size_t head_base) {
-  qkv_blocks<HD, WHICH, 1, T>(blk, dst, src, src_stride, bias, gamma, pe, rope_off, rope_count, rows, token0, tt,
+  qkv_blocks<HD, WHICH, 1, T>(blk, dst, src, src_stride, bias, gamma, pe, rope_off, rope_rows, rows, token0, tt,
                               token_tiles, head_base, 0);
 }
 

@@ -749,7 +749,7 @@ void oracle_qkv_post(uint16_t *q, uint16_t *k, uint16_t *v, const float *raw, co
           qkv_rms_row(row, x, b, which == 0 ? q_norm : k_norm, hd);
           /* rotary (qkv_apply_rope :1210-1231): token = offset + row; rows at or
            * past the count are left as they are */
-          const int token = rope_token_offset + t0 + r;
+          const int64_t token = (int64_t)rope_token_offset + t0 + r;
           if (pe && rope_token_offset >= 0 && rope_token_count > 0 && token < rope_token_count) {
             const float *tp = pe + (size_t)token * (size_t)(hd / 2) * 4u;
             for (int d = 0; d < hd / 2; ++d) {

@@ -354,6 +354,41 @@ def test_post_rope_offset_and_count(orc):
         assert np.array_equal(z[0], plain[0])
 
 
+FAR_OFFSET = 2 ** 31 - 6  # offset + token passes 2^31 within the first tile
+
+
+def test_post_far_rope_offset_rotates_nothing(orc):
+    raw, b, qn, kn, pe = post_inputs(40, 2, 64, 9, rope_tokens=10)
+    far = orc.qkv_post(raw, b, qn, kn, pe, FAR_OFFSET, 10, 40, 2, 64, 2)
+    none = orc.qkv_post(raw, b, qn, kn, None, 0, 0, 40, 2, 64, 2)
+    assert all(np.array_equal(a, c) for a, c in zip(far, none))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [64, 128])
+def test_hb_qkv_far_rope_offset_rotates_nothing(hip, orc, hd):
+    """offset + token as a 32-bit sum would be negative, which is below any count."""
+    tokens, k, heads, tiles = 300, 64, 2, 10
+    cols, size = 3 * heads * hd, heads * h.qkv_head_elems(10, hd)
+    rng = np.random.default_rng(hd)
+    _, b, qn, kn, pe = post_inputs(tokens, heads, hd, 9, rope_tokens=10)
+    x = dev(rng.normal(0, 1, (tokens, k)).astype(np.float32))
+    w = h.f16_prepack(dev(h.permute_f16(rng.normal(0, 0.05, (k, cols)).astype(np.float16).view(np.uint16))), k, cols)
+    raw = h.DeviceBuffer(tokens * cols * 4)
+    h.f16_gemm(raw, x, w, None, tokens, k, cols, cols, 0)
+    h.sync()
+    want = orc.qkv_post(raw.read(np.float32, tokens * cols).reshape(tokens, cols), b, qn, kn, None, 0, 0, tokens, heads,
+                        hd, tiles)
+    post, fused = ([dev(np.zeros(size, np.uint16)) for _ in range(3)] for _ in range(2))
+    h.qkv_post(*post, raw, dev(b), dev(qn), dev(kn), dev(pe), FAR_OFFSET, 10, tokens, heads, hd, tiles, 0)
+    ws = h.DeviceBuffer(h.qkv_gemm_workspace_bytes(tokens, k))
+    h.qkv_gemm(*fused, x, w, dev(b), dev(qn), dev(kn), dev(pe), FAR_OFFSET, 10, tokens, k, heads, hd, tiles, 0, ws)
+    h.sync()
+    for i in range(3):
+        assert np.array_equal(post[i].read(np.uint16, size), want[i])
+        assert np.array_equal(fused[i].read(np.uint16, size), want[i])
+
+
 def test_post_output_offset_keeps_other_tiles(orc):
     raw, bias, qn, kn, _ = post_inputs(20, 1, 64, 9)
     raw2, _, _, _, _ = post_inputs(32, 1, 64, 10)
