@@ -2257,9 +2257,9 @@ bool f16_stream_applies(int m, int k, int n) {
   return 2 * tiles >= cus && (cost < ring_cost || (cost == ring_cost && tiles % cus == 0));
 }
 
+template <int BM, int BN, int S>
 int launch_f16_stream(float *y, const int8_t *a, const int8_t *w, const float *bias, int m, int k, int n, int mode,
                       hipStream_t st) {
-  constexpr int BM = kF16StreamBM, BN = kF16StreamBN, S = kF16StreamStages;
   const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
   const int tiles = tiles_m * tiles_n;
   const int grid = std::min(compute_units(), (tiles + 7) / 8 * 8) / 8 * 8;
@@ -2290,6 +2290,28 @@ bool wide_fits(int k, int n) {
   return (size_t)kWideRows * (size_t)k * 2u < limit && (size_t)kWideRows * (size_t)n * 4u < limit;
 }
 
+// One row of 256-row tiles (193-256 rows) with columns for half of the CUs or
+// more: 64-column tiles that read the weights once, never the ring kernel,
+// whose 64 x 64 tiles read them four times (200x1184x11392 23.9 us against 17.2;
+// at 192 rows the ring stays ahead: 192x4096x10240 31.4 / 35.3).  Up to
+// kStream64Depth values of k the streaming kernel's (its stores overlap the next
+// tile's loads), then the 256 x 64 tiles, two of whose workgroups share a CU.
+// The latter against the former, 323 shapes of n 7000-16384: k 256-400 + 10 %,
+// 400-800 + 7 %, 800-1200 + 3.5 %, 1200-2400 between - 8 and + 7 % (+ 0.5 % on
+// average), 2400-2800 - 2 to - 10 %, 4096 - 12 % (us, 212x544x14208 13.1 / 12.1,
+// 231x1728x11232 22.0 / 20.7, 256x4096x14336 47.5 / 56.4).
+constexpr int kStream64Stages = 7, kStream64Depth = 2400;
+
+bool one_row_of_tiles(int m, int k, int n) {
+  return m > 192 && m <= kWideRows && 2 * ((n + 63) / 64) >= compute_units() && k / 32 >= kStream64Stages - 1 &&
+         wide_fits(k, n);
+}
+
+bool f16_stream64_applies(int m, int k, int n) {
+  return f16_stream_mode() != 0 && one_row_of_tiles(m, k, n) && k < kStream64Depth &&
+         (size_t)n * (size_t)k * 2u < ((size_t)1 << 32);
+}
+
 // The wide tiles to use, or none: predicted microseconds of every candidate
 // after the image pass, as c + rounds * (a + b * k-steps) + f * (output bytes
 // at 5 TB/s), rounds = tiles on the busiest CU; for the ring shapes, several
@@ -2306,6 +2328,7 @@ WideTiles pick_wide(int m, int k, int n) {
   const int force = g_f16_wide.load(std::memory_order_relaxed);
   if (force == 0 || f16_stream_mode() >= 0 || !wide_fits(k, n)) return kWideNone;
   if (force > 0) return (WideTiles)force;
+  if (one_row_of_tiles(m, k, n)) return f16_stream64_applies(m, k, n) ? kWideNone : kWide64;
   const double cus = compute_units(), kt = k / 32, out = (double)m * n * 4.0 / 5e6;
   auto rounds = [&](int bm, int bn) { return std::ceil((double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus); };
   auto wide_us = [&](int bm, int bn, double c, double a, double b, double f, double d = 0.0) {
@@ -2366,6 +2389,25 @@ int launch_wide(WideTiles wide, float *y, const int8_t *a, const int8_t *w, cons
   return launch_wide_mode<0>(wide, y, a, w, bias, m, k, n, st);
 }
 
+// The kernel and the tiles of a product with row-major output that takes the
+// ring path.
+struct RowsPlan {
+  int kernel, bm, bn;
+};
+
+RowsPlan ring_plan(int m, int n) {
+  const RingShape t = kRingShapes[pick_ring_shape(m, n)];
+  return {HB_F16_RING, t.bm, t.bn};
+}
+
+RowsPlan rows_plan(int m, int k, int n) {
+  const WideTiles wide = pick_wide(m, k, n);
+  if (wide != kWideNone) return {HB_F16_WIDE, kWideRows, (int)wide};
+  if (f16_stream64_applies(m, k, n)) return {HB_F16_STREAM, 256, 64};
+  if (f16_stream_applies(m, k, n)) return {HB_F16_STREAM, kF16StreamBM, kF16StreamBN};
+  return ring_plan(m, n);
+}
+
 int launch_ring(float *y, const float *x, const uint16_t *packed, const float *bias, int m, int k, int n, int channels,
                 int mode, void *ws, hipStream_t st) {
   const int mp = (m + 15) / 16 * 16;
@@ -2374,19 +2416,17 @@ int launch_ring(float *y, const float *x, const uint16_t *packed, const float *b
   hipLaunchKernelGGL(f16_pack_a, dim3(pg), dim3(256), 0, st, (uint4 *)ws, x, m, k, mp);
   int rc = hb_check_launch("f16_pack_a");
   if (rc) return rc;
+  const int8_t *a = (const int8_t *)ws, *w = (const int8_t *)packed;
   // The 256-row-tile and streaming kernels write row-major rows only; mode 3
   // takes the ring kernel.
-  const bool rows_out = mode != 3;
-  const WideTiles wide = rows_out ? pick_wide(m, k, n) : kWideNone;
-  if (wide != kWideNone)
-    return launch_wide(wide, y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
-  if (rows_out && f16_stream_applies(m, k, n))
-    return launch_f16_stream(y, (const int8_t *)ws, (const int8_t *)packed, bias, m, k, n, mode, st);
-  const int shape = pick_ring_shape(m, n);
-  const RingShape t = kRingShapes[shape];
-  const int grid = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-  const int8_t *a = (const int8_t *)ws, *w = (const int8_t *)packed;
-  switch (shape) {
+  const RowsPlan p = mode == 3 ? ring_plan(m, n) : rows_plan(m, k, n);
+  if (p.kernel == HB_F16_WIDE) return launch_wide((WideTiles)p.bn, y, a, w, bias, m, k, n, mode, st);
+  if (p.kernel == HB_F16_STREAM && p.bn == 64)
+    return launch_f16_stream<256, 64, kStream64Stages>(y, a, w, bias, m, k, n, mode, st);
+  if (p.kernel == HB_F16_STREAM)
+    return launch_f16_stream<kF16StreamBM, kF16StreamBN, kF16StreamStages>(y, a, w, bias, m, k, n, mode, st);
+  const int grid = ((m + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn);
+  switch (pick_ring_shape(m, n)) {
     case 0:
       hipLaunchKernelGGL((f16_gemm_ring<128, 192, 2, 2, 4>), dim3(grid), dim3(256), 0, st, y, a, w, bias, m, k, n,
                          channels, mode);
@@ -2904,6 +2944,14 @@ int hb_f16_force_wide(int setting) {
   if (setting != -1 && setting != 0 && setting != kWide64 && setting != kWide192 && setting != kWide256)
     return hb_invalid("hb_f16_force_wide setting");
   return g_f16_wide.exchange(setting, std::memory_order_relaxed);
+}
+
+int hb_f16_rows_kernel(int m, int k, int n, int *bm, int *bn) {
+  if (m < 1 || k < 32 || k % 32 || n < 32 || n % 32 || !bm || !bn) return hb_invalid("hb_f16_rows_kernel shape");
+  const RowsPlan p = rows_plan(m, k, n);
+  *bm = p.bm;
+  *bn = p.bn;
+  return p.kernel;
 }
 
 int hb_f16_gemm(float *d_y, const float *d_x, const uint16_t *d_packed, const float *d_bias, int m, int k, int n,

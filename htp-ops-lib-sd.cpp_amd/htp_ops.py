@@ -80,6 +80,7 @@ _SIGNATURES = {
     "hb_w8a8_force_tile": (_c_int, [_c_int]),
     "hb_f16_force_stream": (_c_int, [_c_int]),
     "hb_f16_force_wide": (_c_int, [_c_int]),
+    "hb_f16_rows_kernel": (_c_int, [_c_int, _c_int, _c_int, _c_void_p, _c_void_p]),
     "hb_f16_force_xstream": (_c_int, [_c_int]),
     "hb_f16_force_splitk": (_c_int, [_c_int]),
     "hb_w8a8_gemm_choice": (_c_int, [_c_int, _c_int, _c_int]),
@@ -375,6 +376,16 @@ def f16_force_wide(setting):
     if prev < -1:
         check(prev, "hb_f16_force_wide")
     return prev
+
+
+def f16_rows_kernel(m, k, n):
+    """(kernel, bm, bn) of the F16 ring path for row-major output: "ring",
+    "stream" or "wide" and its tile."""
+    bm, bn = _c_int(), _c_int()
+    rc = lib().hb_f16_rows_kernel(m, k, n, ctypes.addressof(bm), ctypes.addressof(bn))
+    if rc < 0:
+        check(rc, "hb_f16_rows_kernel")
+    return ("ring", "stream", "wide")[rc], bm.value, bn.value
 
 
 def f16_force_xstream(setting):

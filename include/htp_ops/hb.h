@@ -257,8 +257,9 @@ size_t hb_f16_workspace_bytes(int m, int k, int n);
  * -1 restores the automatic choice (the 256-row tiles of hb_f16_force_wide
  * where they are predicted fastest, else the persistent streaming kernel with
  * 256 x 128 tiles where they occupy at least half of the CUs and spread more
- * evenly than the ring kernel's, else the one-tile-per-workgroup ring
- * kernel), 0 keeps the ring
+ * evenly than the ring kernel's, or with 256 x 64 tiles at 193-256 rows with
+ * columns for half of the CUs and k < 2400, else the one-tile-per-workgroup
+ * ring kernel), 0 keeps the ring
  * kernel, 1 runs the streaming kernel wherever it applies (k >= 160).
  * Returns the previous setting.  Results are identical either way.  The
  * environment variable HTP_OPS_AMD_F16_STREAM gives the initial value. */
@@ -272,6 +273,14 @@ int hb_f16_force_stream(int setting);
  * Returns the previous setting.  Results are identical for every setting.  No
  * counterpart in the reference. */
 int hb_f16_force_wide(int setting);
+
+/* The kernel that hb_f16_gemm_ws takes for row-major output (modes 0-2) where
+ * it takes neither a split-K path nor the activation-streaming kernel and the
+ * ring path applies, with the settings above; *bm x *bn is its tile.  For
+ * tests and tuning, no counterpart in the reference; HB_E_INVAL on a bad
+ * shape. */
+enum { HB_F16_RING = 0, HB_F16_STREAM = 1, HB_F16_WIDE = 2 };
+int hb_f16_rows_kernel(int m, int k, int n, int *bm, int *bn);
 
 /* Pins the activation-streaming F16 kernel (f16_gemm_xstream: the fp32
  * activations read once, converted in registers, for many rows and few

@@ -572,6 +572,8 @@ def test_f16_ring_matches_tiles(hip, orc, m, k, n, mode, bias, check_oracle):
     (2048, 1536, 1152, 0, True, False),   # long k, few tiles
     (333, 224, 2080, 2, True, True),      # n % 128 == 32: a last tile of one column pair, its bias clamped
     (256, 256, 8192, 1, True, False),     # one 256-row tile: 256 x 64 streaming tiles
+    (193, 192, 8224, 0, True, True),      # the least k of those tiles, n % 64 == 32, most of the last rows past m
+    (240, 2368, 8160, 2, False, False),   # the longest k, a last tile of 32 columns
 ])
 def test_f16_stream_matches_ring(hip, orc, m, k, n, mode, bias, check_oracle):
     """The persistent streaming F16 kernel gives the same bits as the ring
