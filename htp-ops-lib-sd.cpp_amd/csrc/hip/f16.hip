@@ -2312,45 +2312,62 @@ bool f16_stream64_applies(int m, int k, int n) {
          (size_t)n * (size_t)k * 2u < ((size_t)1 << 32);
 }
 
-// The wide tiles to use, or none: predicted microseconds of every candidate
-// after the image pass, as c + rounds * (a + b * k-steps) + f * (output bytes
-// at 5 TB/s), rounds = tiles on the busiest CU; for the ring shapes, several
-// workgroups to a CU (also two of the 256 x 64 tiles), d * k-steps besides.  Fitted to
-// 83 shapes from 200 to 4173 rows, k 768-8192, n 768-14336 (each kernel forced
-// on each shape; errors 3-5 % on average, 15 % at most).  The choice is within
-// 1 % of the fastest candidate on average, 7 % at most, and against the ring
-// and streaming kernels alone, us before / after: 2048x4096x14336 230 / 202,
-// 4173x1536x6144 108 / 94, 1024x4096x14336 116 / 102, 2048x8192x2048 119 / 89,
-// 4173x8192x2048 221 / 162, 3000x4608x1152 74 / 55, 4096x4096x1024 71 / 58,
-// 1101x2048x8192 61 / 46, 4173x768x3072 39 / 33.  They must lead by 2 %, below
-// which the measurements do not tell them apart.
+// Predicted microseconds of a kernel after the image pass: c + rounds * (round
+// + step * k-steps) + out * (output bytes at 5 TB/s) + depth * k-steps, rounds =
+// tiles on the busiest CU (64 x 64 ring tiles, of which four share a CU: tiles
+// per CU, not rounded).  Fitted to 1389 shapes of 129 to 16384 rows, k 64-8192,
+// n 512-14336, each kernel forced on each shape (profiles/f16_rows_tiles.csv);
+// errors 4-7 % on average.
+struct UsFit {
+  double c, round, step, out, depth;
+
+  double us(double rounds, double kt, double out_us) const {
+    return c + rounds * (round + step * kt) + out * out_us + depth * kt;
+  }
+};
+constexpr UsFit kRingFit[3] = {
+    {5.11, 1.35, 0.378, 0.796, -0.128}, {5.79, 2.22, 0.273, 0.374, -0.069}, {6.36, 0.0, 0.074, 0.571, 0.113}};
+constexpr UsFit kStreamFit = {6.35, 2.33, 0.334, 0.678, 0.0};
+constexpr UsFit kWide64Fit = {7.71, 0.91, 0.216, 0.540, 0.0};
+constexpr UsFit kWide192Fit = {4.79, 9.08, 0.449, 0.262, 0.0};
+constexpr UsFit kWide256Fit = {2.24, 12.11, 0.520, 0.193, 0.0};
+
+// The wide tiles to use, or none: the fastest by prediction, if it leads the
+// ring or streaming kernel by kWideLead, below which the predictions do not
+// tell them apart; the 64-column tiles also only where they fill three quarters
+// of a round of CUs (fewer gain 1 % on average and lose up to 17 %).  Over the
+// shapes above that is 3.4 % faster than those two kernels alone on average,
+// slower by more than 2 % on 7 of them (at most 13 %, 4141x128x8160: stores) and
+// 1.5 % behind the fastest candidate of each.  us, before the wide tiles /
+// after: 2048x4096x14336 230 / 202, 4173x1536x6144 108 / 94, 1024x4096x14336
+// 116 / 102, 4173x8192x2048 221 / 162, 3000x4608x1152 74 / 55, 4096x4096x1024
+// 71 / 58.
+constexpr double kWideLead = 0.07, kWide64Fill = 0.75;
+
 WideTiles pick_wide(int m, int k, int n) {
   const int force = g_f16_wide.load(std::memory_order_relaxed);
   if (force == 0 || f16_stream_mode() >= 0 || !wide_fits(k, n)) return kWideNone;
   if (force > 0) return (WideTiles)force;
   if (one_row_of_tiles(m, k, n)) return f16_stream64_applies(m, k, n) ? kWideNone : kWide64;
-  const double cus = compute_units(), kt = k / 32, out = (double)m * n * 4.0 / 5e6;
-  auto rounds = [&](int bm, int bn) { return std::ceil((double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus); };
-  auto wide_us = [&](int bm, int bn, double c, double a, double b, double f, double d = 0.0) {
-    return c + rounds(bm, bn) * (a + b * kt) + f * out + d * kt;
-  };
-  static const double kRingFit[3][4] = {
-      {13.9, -0.61, 0.4454, -0.2597}, {6.5, 2.40, 0.2598, -0.1467}, {3.7, 0.73, 0.0619, 0.0674}};
+  const double cus = compute_units(), kt = k / 32, out_us = (double)m * n * 4.0 / 5e6;
+  auto per_cu = [&](int bm, int bn) { return (double)((m + bm - 1) / bm) * ((n + bn - 1) / bn) / cus; };
+  auto predict = [&](const UsFit &f, int bm, int bn) { return f.us(std::ceil(per_cu(bm, bn)), kt, out_us); };
   const int shape = pick_ring_shape(m, n);
-  const double *f = kRingFit[shape];
-  double present = f[0] + rounds(kRingShapes[shape].bm, kRingShapes[shape].bn) * (f[1] + f[2] * kt) + f[3] * kt;
-  if (f16_stream_applies(m, k, n)) present = wide_us(256, 128, 1.75, 5.46, 0.277, 0.90);
+  const RingShape ring = kRingShapes[shape];
+  double present = ring.bm == 64 ? kRingFit[shape].us(per_cu(ring.bm, ring.bn), kt, out_us)
+                                 : predict(kRingFit[shape], ring.bm, ring.bn);
+  if (f16_stream_applies(m, k, n)) present = predict(kStreamFit, kF16StreamBM, kF16StreamBN);
   WideTiles best = kWideNone;
-  double best_us = 0.98 * present;
+  double best_us = (1.0 - kWideLead) * present;
   auto consider = [&](WideTiles t, double us) {
     if (us < best_us) {
       best_us = us;
       best = t;
     }
   };
-  consider(kWide64, wide_us(256, 64, 6.68, -0.77, 0.220, 1.14, -0.029));
-  consider(kWide192, wide_us(256, 192, -2.11, 13.31, 0.391, 0.61));
-  consider(kWide256, wide_us(256, 256, -5.85, 17.16, 0.490, 0.58));
+  if (per_cu(kWideRows, 64) >= kWide64Fill) consider(kWide64, predict(kWide64Fit, kWideRows, 64));
+  consider(kWide192, predict(kWide192Fit, kWideRows, 192));
+  consider(kWide256, predict(kWide256Fit, kWideRows, 256));
   return best;
 }
 

@@ -24,3 +24,19 @@ def test_one_row_of_256_row_tiles(m, k, n, want):
 @pytest.mark.parametrize("m,k,n", [(192, 1184, 11392), (200, 160, 11392), (200, 1184, 8064)])
 def test_one_row_of_256_row_tiles_outside(m, k, n):
     assert h.f16_rows_kernel(m, k, n)[:2] != ("stream", 256)
+
+
+@pytest.mark.parametrize("m,k,n,want", [
+    (3852, 672, 5984, "stream"),   # us: 52.8, 56.8 on 256 x 64 tiles
+    (4589, 544, 7584, "stream"),   # 70.2 / 74.6
+    (14468, 608, 3520, "stream"),  # 99 / 112
+    (2140, 1376, 1056, "ring"),    # 22.7 / 26.5
+    (1920, 2592, 1184, "ring"),    # 31.8 / 33.8
+    (2181, 1664, 928, "ring"),     # 23.7 / 27.3
+    (4173, 1536, 6144, "wide"),
+    (4173, 6144, 1536, "stream"),
+    (2048, 4096, 14336, "wide"),
+    (4096, 4096, 1024, "wide"),
+])
+def test_predicted_tiles(m, k, n, want):
+    assert h.f16_rows_kernel(m, k, n)[0] == want
