@@ -2315,7 +2315,7 @@ bool f16_stream64_applies(int m, int k, int n) {
 // Predicted microseconds of a kernel after the image pass: c + rounds * (round
 // + step * k-steps) + out * (output bytes at 5 TB/s) + depth * k-steps, rounds =
 // tiles on the busiest CU (64 x 64 ring tiles, of which four share a CU: tiles
-// per CU, not rounded).  Fitted to 1389 shapes of 129 to 16384 rows, k 64-8192,
+// per CU, not rounded).  Fitted to 1389 shapes of 94 to 16384 rows, k 64-8192,
 // n 512-14336, each kernel forced on each shape (profiles/f16_rows_tiles.csv);
 // errors 4-7 % on average.
 struct UsFit {
@@ -2504,19 +2504,20 @@ int ring_slices(int m, int k, int n, int &kps) {
 // (f16_rows_splitk) or an fp16 image of them: at most one workgroup per CU (a
 // second one has to share the CU's operand rate, of which fp32 rows take
 // half more), and no more k-steps a slice than the image pass pays for (its
-// launch about 20, its traffic 0.9 per MB of x; the line lies between the
-// pairs below).  Measured, us, image / rows, same slices (k-steps each):
+// launch about 16, its traffic 1.2 per MB of x; the line by 444 shapes of both
+// forms, on which its choice is 0.3 % behind the faster form on average, 7 % at
+// most).  Measured, us, image / rows, same slices (k-steps each):
 // 1024x5760x640 (30) 29.1 / 26.7, 2048x4608x512 (36) 34.8 / 29.0, 900x10240x512
 // (40) 35.8 / 30.5, 2048x11520x256 (45) 53.0 / 34.5, 700x5760x640 (23) 25.4 /
-// 22.9, 77x4096x4096 (16) 17.2 / 14.9, 77x5120x3072 (20) 17.0 / 16.0,
-// 250x2048x1024 (8) 16.2 / 12.3; left on the image: 171x6144x1536 (24) 19.4 /
-// 20.8, 171x8192x2048 (32) 23.8 / 26.2, 120x8640x960 (34) 22.5 / 23.8,
-// 500x6144x1536 (39) 27.9 / 30.4, 512x11520x1280 (60) 39.3 / 41.1,
-// 128x10240x4096 (40) 27.9 / 30.8.
+// 22.9, 77x4096x4096 (16) 17.2 / 14.9, 250x2048x1024 (8) 16.2 / 12.3; left on
+// the image: 171x6144x1536 (24) 19.4 / 20.8, 171x8192x2048 (32) 23.8 / 26.2,
+// 362x7232x1056 (29) 26.8 / 30.3, 120x8640x960 (34) 22.5 / 23.8, 500x6144x1536
+// (39) 27.9 / 30.4, 512x11520x1280 (60) 39.3 / 41.1, 128x10240x4096 (40) 27.9 /
+// 30.8, and 77x5120x3072 (20) 17.0 / 16.0.
 bool splitk_rows(int m, int k, int n) {
   int kps = 0;
   const int slices = ring_slices(m, k, n, kps);
-  return tiles128(m, n) * slices <= compute_units() && kps <= 20.0 + 0.9e-6 * 4.0 * m * (double)k;
+  return tiles128(m, n) * slices <= compute_units() && kps <= 16.0 + 1.2e-6 * 4.0 * m * (double)k;
 }
 
 // From 257 rows and k >= 2048: the split-K ring path where 128 x 128 tiles

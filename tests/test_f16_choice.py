@@ -40,3 +40,18 @@ def test_one_row_of_256_row_tiles_outside(m, k, n):
 ])
 def test_predicted_tiles(m, k, n, want):
     assert h.f16_rows_kernel(m, k, n)[0] == want
+
+
+@pytest.mark.parametrize("m,k,n,slices,image", [
+    (362, 7232, 1056, 8, True),   # us: image 26.8, fp32 rows 30.3
+    (294, 6304, 96, 8, True),     # 17.7 / 18.6
+    (500, 6144, 1536, 5, True),
+    (1024, 5760, 640, 6, False),  # 29.1 / 26.7
+    (2048, 4608, 512, 4, False),
+])
+def test_splitk_form(m, k, n, slices, image):
+    """From 257 rows the split-K path's workspace holds the fp16 image only
+    where that form runs."""
+    mp = (m + 15) // 16 * 16
+    need = slices * mp * n * 4 + (mp * k * 2 + 255) // 256 * 256 * image
+    assert h.f16_workspace_bytes(m, k, n) == max(need, mp * k * 2)
