@@ -3048,6 +3048,38 @@ int hb_qkv_gemm_unsplit(int tokens, int input_dim, int n_heads, int head_dim) {
   return ring_splitk_mode() != 1 && ring_before_splitk(tokens, input_dim, n);
 }
 
+// Parts that may be fused: 512 tokens or more, or a product that
+// hb_f16_gemm_ws would not split over K (the results are the same either way).
+// With heads of 64 they always are: at 129-511 tokens as fast as the GEMM and
+// hb_qkv_post or up to 30 % faster.  Heads of 128 take 256 x 128 tiles, one
+// workgroup to a CU: a launch costs whole rounds of them however few rows it
+// holds, and a part of fewer than 384 tokens by itself about 0.8 of a round
+// without the fusion.  Measured, us, 24 heads, input 3072, separate GEMM /
+// fused: 129 tokens 35.2 / 46.4, 256 40.1 / 51.8, 320 44.3 / 52.3, 384 56.2 /
+// 52.9, 511 54.6 / 53.5; image + text, separate / one launch: 256 + 160 70.3 /
+// 53.6 (one round), 256 + 300 79.9 / 57.8, 256 + 600 93.7 / 105.2 (two rounds
+// where 600 tokens alone take one), 640 + 200 93.5 / 105.9.
+int hb_qkv_gemm_plan(const int *tokens, int n_parts, int input_dim, int n_heads, int head_dim) {
+  if (!tokens || n_parts < 1 || n_parts > 2 || n_heads <= 0 || (head_dim != 64 && head_dim != 128))
+    return hb_invalid("hb_qkv_gemm_plan arguments");
+  if ((n_heads * head_dim) % 128 || !wide_fits(input_dim, 32)) return 0;
+  int plan = 0, can = 0, bands = 0;
+  const long long columns = 3 * n_heads, cus = compute_units();
+  auto rounds = [&](long long b) { return (b * columns + cus - 1) / cus; };
+  long long tenths = 0;  // of a round, by separate launches
+  for (int i = 0; i < n_parts; ++i) {
+    const int b = (tokens[i] + kWideRows - 1) / kWideRows;
+    bands += b;
+    if (tokens[i] < 512 && !hb_qkv_gemm_unsplit(tokens[i], input_dim, n_heads, head_dim)) continue;
+    ++can;
+    const bool alone = head_dim == 64 || tokens[i] >= 384;
+    if (alone) plan |= 1 << i;
+    tenths += alone ? 10 * rounds(b) : 8;
+  }
+  if (can == 2 && (head_dim == 64 || 10 * rounds(bands) <= tenths)) plan |= 4;
+  return plan;
+}
+
 int hb_qkv_gemm(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const float *d_x, const uint16_t *d_packed,
                 const float *d_bias, const float *d_q_norm, const float *d_k_norm, const float *d_pe, int rope_offset,
                 int rope_count, int tokens, int input_dim, int n_heads, int head_dim, int token_tiles, int out_offset,

@@ -984,22 +984,23 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     if (built) extra_us += (now_seconds() - t0) * 1e6;
   }
 
-  /* A part of 512 tokens or more, or one whose product the F16 GEMM would not
-   * split over K (from 129 tokens, so that the results are the same either
-   * way), runs the GEMM with the post-processing in its epilogue; the others
-   * the GEMM into scratch, then hb_qkv_post.  Two fused parts are one launch
-   * where no input needs a realigned copy (those share scratch slots). */
+  /* Parts with the post-processing in the GEMM's epilogue by hb_qkv_gemm_plan;
+   * the others the GEMM into scratch, then hb_qkv_post.  Two parts are one
+   * launch only where no input needs a realigned copy (those share scratch
+   * slots). */
+  const int tokens[2] = {parts[0].tokens, n_parts == 2 ? parts[1].tokens : 0};
+  const int plan = hb_qkv_gemm_plan(tokens, n_parts, input_dim, n_heads, head_dim);
+  if (plan < 0) return -5;
+  const int joint = (plan & 4) && qkv_part_in_place(&parts[0]) && qkv_part_in_place(&parts[1]);
   int fused[2] = {0, 0};
   size_t ws_max = 0, ws_sum = 0;
   for (int i = 0; i < n_parts; ++i) {
-    fused[i] = (ncols / 3) % 128 == 0 &&
-               (parts[i].tokens >= 512 || hb_qkv_gemm_unsplit(parts[i].tokens, input_dim, n_heads, head_dim));
+    fused[i] = joint || (plan >> i & 1);
     const size_t b = fused[i] ? hb_qkv_gemm_workspace_bytes(parts[i].tokens, input_dim)
                               : hb_f16_workspace_bytes(parts[i].tokens, input_dim, ncols);
     ws_max = b > ws_max ? b : ws_max;
     ws_sum += b;
   }
-  const int joint = n_parts == 2 && fused[0] && fused[1] && qkv_part_in_place(&parts[0]) && qkv_part_in_place(&parts[1]);
   if (joint) ws_max = ws_sum;
   int raw_tokens = 0;
   for (int i = 0; i < n_parts; ++i)

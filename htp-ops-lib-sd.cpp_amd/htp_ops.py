@@ -108,6 +108,7 @@ _SIGNATURES = {
     "hb_qkv_gemm_parts": (_c_int, [_c_void_p] * 4 + [_c_int, _c_void_p] + [_c_int] * 5 + [_c_void_p, _c_size_t,
                                                                                         _c_void_p]),
     "hb_qkv_gemm_unsplit": (_c_int, [_c_int] * 4),
+    "hb_qkv_gemm_plan": (_c_int, [_c_void_p] + [_c_int] * 4),
     "hb_model_aux_ws": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p] + [_c_int] * 9 +
                         [ctypes.c_float, _c_void_p, _c_size_t, _c_void_p]),
 }
@@ -752,6 +753,15 @@ def qkv_gemm_parts(q_dev, k_dev, v_dev, parts, pe_dev, rope_count, input_dim, n_
     check(lib().hb_qkv_gemm_parts(q_dev.ptr, k_dev.ptr, v_dev.ptr, ctypes.addressof(arr), len(parts), pe, rope_count,
                                   input_dim, n_heads, head_dim, token_tiles, workspace.ptr, workspace.nbytes, stream),
           "hb_qkv_gemm_parts")
+
+
+def qkv_gemm_plan(tokens, input_dim, n_heads, head_dim):
+    """hb_qkv_gemm_plan of one or two token counts."""
+    arr = (_c_int * len(tokens))(*tokens)
+    rc = lib().hb_qkv_gemm_plan(ctypes.addressof(arr), len(tokens), input_dim, n_heads, head_dim)
+    if rc < 0:
+        check(rc, "hb_qkv_gemm_plan")
+    return rc
 
 
 def matmul_params(out, act, wgt, m, k, n, with_elapsed=False):

@@ -405,6 +405,12 @@ int hb_qkv_gemm_parts(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const hb_qkv_
  * workspace) does not split K, so that hb_qkv_gemm_parts gives the same bits
  * as hb_f16_gemm_ws followed by hb_qkv_post. */
 int hb_qkv_gemm_unsplit(int tokens, int input_dim, int n_heads, int head_dim);
+/* The faster form of one or two parts of these token counts: bit i, part i by
+ * itself as hb_qkv_gemm (else hb_f16_gemm_ws and hb_qkv_post); 4, both parts as
+ * one hb_qkv_gemm_parts.  Only parts that hb_qkv_gemm takes, and below 512
+ * tokens only those whose results are the same bits either way.  HB_E_INVAL on
+ * bad arguments. */
+int hb_qkv_gemm_plan(const int *tokens, int n_parts, int input_dim, int n_heads, int head_dim);
 
 #ifdef __cplusplus
 }

@@ -505,6 +505,28 @@ int main(int, char **v) {
 """
 
 
+@pytest.mark.parametrize("tokens,k,heads,hd,plan", [
+    ((160, 77), 3072, 24, 128, 0),     # us: separate 66.2, the image part fused 76.2
+    ((256, 77), 3072, 24, 128, 0),     # 69.8 / 80.9
+    ((300,), 4096, 24, 128, 0),
+    ((383,), 3072, 24, 128, 0),
+    ((384,), 3072, 24, 128, 1),
+    ((256, 160), 3072, 24, 128, 4),    # one round of tiles
+    ((256, 600), 3072, 24, 128, 2),    # 93.7, one launch of two rounds 105.2
+    ((640, 200), 3072, 24, 128, 1),
+    ((512, 512), 3072, 24, 128, 7),
+    ((256, 4096), 3072, 24, 128, 6),
+    ((256, 4096), 1536, 24, 64, 7),
+    ((256, 300), 1920, 30, 64, 7),
+    ((256, 77), 2432, 38, 64, 1),
+    ((32, 1), 1536, 24, 64, 0),
+    ((4096,), 1 << 23, 24, 64, 0),     # past the fused kernel's 32-bit offsets
+])
+def test_qkv_plan(tokens, k, heads, hd, plan):
+    """Which parts take the fused kernel, on 256 CUs."""
+    assert h.qkv_gemm_plan(tokens, k, heads, hd) == plan
+
+
 def test_rotary_rows_read(tmp_path):
     """The fused kernels load a rotary matrix for every lane of a 32-token
     tile: no row past the last rotated token is read, whatever the offsets of
