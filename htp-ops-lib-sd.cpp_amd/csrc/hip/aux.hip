@@ -381,9 +381,13 @@ __global__ __launch_bounds__(kAuxThreads) void aux_group_norm_chunk(float *__res
 // where the memory-side cache holds it (aux_group_norm_chunk at 128 channels
 // of 512 x 512: 25 us for the statistics pass and 47 for the output pass, in
 // either order), so 512 KB held per CU save a third of the traffic.  32 groups
-// without parameters, both passes -> this kernel, microseconds: 512 x 128^2
-// 21.4 -> 18.3, 256 x 256^2 39.0 -> 29.4, 256 x 320^2 59.3 -> 44.1, 128 x 512^2
-// 72.2 -> 59.8 (268 MB at 4.5 TB/s; a copy of that size reaches 5.1).
+// with parameters and SiLU, both passes -> this kernel, microseconds: 512 x
+// 128^2 21.5 -> 18.9, 256 x 256^2 39.1 -> 30.1, 256 x 320^2 57.2 -> 43.7, 128 x
+// 512^2 72.3 -> 55.3 (268 MB at 4.9 TB/s; a copy of that size reaches 5.1); x
+// written by the launch before, 128 x 512^2 67.9 -> 50.5.  Rows of T float4s past
+// a piece are skipped: a form holds up to twice the piece, and working them out
+// unstored took it behind the two passes (256 x 33175: 29.5 us in two passes,
+// 32.5 with them, 25.1 without).
 //
 // The exchange: parts holds one slot per (task, piece, sum) that a fill kernel
 // set to kGnEmpty; every workgroup stores its two sums with device-scope
@@ -529,12 +533,14 @@ __global__ __launch_bounds__(kGnThreads) void aux_group_norm_resident(
   const int last = quads - 1;  // lanes past the piece compute some value of the group
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
+    if (u * T >= have) break;
     const hb_f32x4 o = out.value(v[u], min(v0 + u * T + t, last));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(hb_u32x4, o), row(yp, u), at, 0, 2);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int u = 0; u < NL; ++u) {
+    if ((NV + u) * T >= have) break;
     const float4 l = held_lds[u * T + t];
     const hb_f32x4 o = out.value(hb_f32x4{l.x, l.y, l.z, l.w}, min(v0 + (NV + u) * T + t, last));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(hb_u32x4, o), row(yp, NV + u), at, 0, 2);
@@ -833,7 +839,7 @@ struct ResidentPlan {
 };
 // Below 8 M values the two passes are as fast: the second read comes from the
 // XCDs' own L2s, and the exchange costs about 3 us (320 x 128^2, 5.2 M values:
-// 14.3 us in both forms; 512 x 128^2, 8.4 M: 20.1 in two passes, 18.3 here).
+// 14.3 us in both forms; 512 x 128^2, 8.4 M: 21.5 in two passes, 18.9 here).
 constexpr int64_t kGnResidentMin = 8 << 20;
 constexpr int kGnHeld = 32;  // float4s per thread that registers and LDS hold
 
@@ -951,9 +957,9 @@ extern "C" int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, c
           hipLaunchKernelGGL(aux_group_norm_clear, dim3((slots + 255) / 256), dim3(256), 0, st,
                              (unsigned long long *)d_workspace, slots);
           if (int rc = hb_check_launch("aux_group_norm_clear")) return rc;
-          // The fewest registers and the least LDS that hold the piece: 26
-          // float4s take 49.7 us in the largest form and 44.1 in their own
-          // (256 x 320^2), 20 take 43.2 and 39.1 (256 x 80000 values).
+          // The fewest registers and the least LDS that hold the piece: in
+          // the largest form 12 float4s take 26.3 us instead of 24.3, 20 take
+          // 38.0 instead of 36.5, 26 the same (256 channels).
           if (rp.per_thread <= 8)
             launch_resident<8, 0>(rp, d_y, d_x, d_w, d_b, ws, len, tasks, channels, spatial, groups, eps, activation, st);
           else if (rp.per_thread <= 16)
