@@ -856,8 +856,12 @@ ResidentPlan resident_plan(int tasks, int len, int chunks) {
 }
 
 // How long a workgroup of the resident form waits for another's sums before
-// it computes them itself, in 100 MHz ticks (2 ms; hb_group_norm_spin).
-std::atomic<int> g_gn_spin{200000};
+// it computes them itself, in 100 MHz ticks (hb_group_norm_spin): 100 us, twice
+// the longest launch, so that a call whose workgroups find no CU (another
+// stream's kernel holds it, or a CU mask) is not held up for much longer than
+// two passes take.  Beside 30 products of all CUs on another stream waits of 10,
+// 100 and 2000 us take the same time, 100-119 us a call (two passes 205).
+std::atomic<int> g_gn_spin{10000};
 
 template <int NV, int NL>
 void launch_resident(const ResidentPlan &p, float *y, const float *x, const float *w, const float *b, void *ws, int len,

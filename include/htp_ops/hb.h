@@ -350,7 +350,7 @@ int hb_model_aux_ws(float *d_y, const float *d_x, const float *d_w, const float 
                     int channels, int spatial, int groups, int batch, int other_count, int activation, float eps,
                     void *d_workspace, size_t workspace_bytes, hb_stream s);
 
-/* Sets how long (100 MHz ticks, 200000 by default) a workgroup of the
+/* Sets how long (100 MHz ticks, 10000 by default) a workgroup of the
  * one-read group norm waits for another workgroup's sums before it computes
  * them itself; returns the previous value.  A test hook: results do not
  * depend on it. */

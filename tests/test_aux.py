@@ -371,6 +371,14 @@ def test_aux_group_norm_split_gpu(hip, orc, batch, channels, groups, spatial, af
     np.testing.assert_allclose(got, want, rtol=rtol, atol=atol)
 
 
+def test_aux_group_norm_wait_is_a_few_launches_long():
+    """Workgroups of the one-read group norm wait for each other at most a few
+    times the longest launch (60 us; in 100 MHz ticks)."""
+    prev = h.lib().hb_group_norm_spin(1)
+    assert h.lib().hb_group_norm_spin(prev) == 1
+    assert 6000 <= prev <= 20000
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,channels,groups,spatial,affine,act,kind", [
     (1, 512, 32, 16384, True, 1, "normal"),    # 8 M values, the smallest taken: 8 float4 per thread exactly
