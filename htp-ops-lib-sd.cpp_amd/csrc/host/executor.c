@@ -263,8 +263,10 @@ static double event_ms(const event_set *ev, int a, int b) {
  * while that stamp is not written yet (the GPU is still busy, so no idle time
  * counts) and nothing else, such as a realigning copy, was queued since.
  * Measured: 16 requests of one row, 4096 -> 14336, 302 -> 209 us; a DiT block
- * of nine requests 440 -> 390 us.  A request by itself keeps two events: the
- * stamps' launches lengthen its chain (23.4 against 25.6 us). */
+ * of nine requests 440 -> 390 us.  A request by itself, or one that completes
+ * before the next starts (a host-resident output), keeps two events: the
+ * stamps' launches lengthen its chain (23.4 against 25.6 us; two requests of
+ * 77x768 with outputs on the host 57.6 against 59.4). */
 enum { kStampSlots = 256 };
 static volatile uint64_t *g_stamps;
 static double g_stamp_us;        /* microseconds per tick */
@@ -297,8 +299,9 @@ static int stamp_take(int *slot, hb_stream s) {
   return hb_stamp((uint64_t *)&g_stamps[*slot], s) == HB_OK ? 0 : HB_E_HIP;
 }
 
-static int span_begin(op_span *sp, hb_stream s) {
-  sp->stamped = g_in_message && g_message_requests > 1;
+/* deferrable: the request need not complete before the next one starts. */
+static int span_begin(op_span *sp, int deferrable, hb_stream s) {
+  sp->stamped = g_in_message && g_message_requests > 1 && deferrable;
   if (!sp->stamped) {
     if (events_open(&sp->ev, 2)) {
       events_close(&sp->ev);
@@ -328,7 +331,8 @@ static int span_end(op_span *sp, hb_stream s) {
 
 /* Hands slots and events back after a stream synchronisation (those of
  * deferred requests stay taken until their flush). */
-static void span_release(void) {
+static void span_release(op_span *sp) {
+  if (sp && !sp->stamped) events_close(&sp->ev);
   if (g_deferred_n == 0) g_stamp_next = g_event_next = 0;
   g_stamp_edge = -1;
 }
@@ -391,13 +395,13 @@ static int flush_deferred_locked(void) {
     }
   }
   g_deferred_n = 0;
-  span_release();
+  span_release(NULL);
   return rc == HB_OK ? 0 : -5;
 }
 
 /* Completes the queued work of one request: defers it when the message
  * allows, else synchronises and writes elapsed_us. */
-static int complete(const op_span *sp, uint8_t *elapsed_dst, double extra_us, int deferrable) {
+static int complete(op_span *sp, uint8_t *elapsed_dst, double extra_us, int deferrable) {
   if (g_in_message && deferrable && g_deferred_n < kMaxDeferred) {
     deferred_op *d = &g_deferred[g_deferred_n++];
     d->elapsed_dst = elapsed_dst;
@@ -412,7 +416,7 @@ static int complete(const op_span *sp, uint8_t *elapsed_dst, double extra_us, in
     const int32_t us = (int32_t)(span_us(sp) + extra_us);
     memcpy(elapsed_dst, &us, sizeof(us));
   }
-  span_release();
+  span_release(sp);
   return rc == HB_OK ? 0 : -5;
 }
 
@@ -623,7 +627,7 @@ static int exec_w8a8(uint8_t *payload, size_t payload_size) {
     if (cpu_output && ctl.is_device) free(hc);
     return -5;
   }
-  int hrc = split ? hb_event_record(ev.e[0], s) : span_begin(&span, s);
+  int hrc = split ? hb_event_record(ev.e[0], s) : span_begin(&span, out.is_device, s);
   /* A plain request runs through hb_w8a8_linear, which takes the one-launch
    * kernels that quantize their own rows where the shape allows (m == 1,
    * 2-4 rows, 5-128 rows with short K) and quantize + GEMM otherwise; all
@@ -700,7 +704,7 @@ static int exec_w8a8(uint8_t *payload, size_t payload_size) {
   const double gemm_ms = split ? event_ms(&ev, 1, 2) : span_us(&span) * 1e-3;
   const double out_ms = split ? event_ms(&ev, 2, 3) : 0.0;
   if (split) events_close(&ev);
-  else span_release();
+  else span_release(&span);
 
   if (cpu_output && ctl.is_device) {
     /* an HBM-resident control block is written once, after every batch */
@@ -798,7 +802,7 @@ static int run_f16(int kind, int qk0_type, htp_view *out, htp_view *act, htp_vie
   void *ws = ws_bytes ? htp_executor_scratch(4, ws_bytes) : NULL;
   if (ws_bytes && !ws) return -5;
   op_span span;
-  int hrc = span_begin(&span, s);
+  int hrc = span_begin(&span, out->is_device, s);
   if (!hrc)
     hrc = direct ? hb_qk0_gemm_ws(y, x, (const uint8_t *)packed, m, k, n, qk0_type, ws, ws_bytes, s)
                  : hb_f16_gemm_ws(y, x, (const uint16_t *)packed, b, m, k, n, channels, mode, ws, ws_bytes, s);
@@ -1017,6 +1021,7 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     d_pe = (const float *)aligned_input(pe, 16, 7, s);
     if (!d_pe) return -5;
   }
+  const int device_outputs = out[0].is_device && out[1].is_device && out[2].is_device;
   op_span span;
   int hrc = 0;
   hb_qkv_part joined[2];
@@ -1039,13 +1044,13 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
       const hb_qkv_part j = {x, (const uint16_t *)packed[i], b, qn, kn, p->rope_offset, p->tokens, p->out_offset};
       joined[i] = j;
       if (i == 0) continue;
-      hrc = span_begin(&span, s);
+      hrc = span_begin(&span, device_outputs, s);
       if (!hrc)
         hrc = hb_qkv_gemm_parts(dst[0], dst[1], dst[2], joined, 2, d_pe, rope_count, input_dim, n_heads, head_dim,
                                 token_tiles, ws, ws_max, s);
       continue;
     }
-    if (i == 0) hrc = span_begin(&span, s);
+    if (i == 0) hrc = span_begin(&span, device_outputs, s);
     if (!hrc && fused[i])
       hrc = hb_qkv_gemm(dst[0], dst[1], dst[2], x, (const uint16_t *)packed[i], b, qn, kn, d_pe, p->rope_offset,
                         rope_count, p->tokens, input_dim, n_heads, head_dim, token_tiles, p->out_offset, ws, ws_max,
@@ -1062,7 +1067,6 @@ static int run_qkv(htp_view out[3], qkv_part *parts, int n_parts, htp_view *pe, 
     if ((void *)dst[i] != out[i].dev) hrc = queue_copy(out[i].dev, dst[i], out[i].bytes, s);
   if (hrc) return hrc == HB_E_INVAL ? -1 : -5;
   for (int i = 0; i < 3; ++i) htp_registry_touch(out[i].fd, out[i].offset, out[i].bytes);
-  const int device_outputs = out[0].is_device && out[1].is_device && out[2].is_device;
   if (complete(&span, elapsed_dst, extra_us, device_outputs)) return -5;
   for (int i = 0; i < 3; ++i)
     if (stage_out(&out[i], s)) return -5;
@@ -1276,7 +1280,7 @@ static int exec_model_aux(uint8_t *payload, size_t payload_size) {
   void *ws = ws_bytes ? htp_executor_scratch(4, ws_bytes) : NULL;
   if (ws_bytes && !ws) return -5;
   op_span span;
-  int hrc = span_begin(&span, s);
+  int hrc = span_begin(&span, out.is_device, s);
   if (!hrc)
     hrc = hb_model_aux_ws(y, x, w, b, p.mode, p.count, p.width, p.channels, p.spatial, p.groups, p.batch,
                           p.other_count, p.activation, p.eps, ws, ws_bytes, s);
