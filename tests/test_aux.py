@@ -510,6 +510,33 @@ def test_aux_gated_gpu(hip, orc, act, rows, width, channels):
 
 
 @pytest.mark.gpu
+def test_aux_sigmoid_has_the_library_sequences_bits(hip):
+    """SiLU at every float of either sign from 2^-26 to 128 (the exponential is
+    1 / 2 ... 1 below, clamped above): the bits of exp2f and an IEEE division,
+    here torch's exp2 on the same device and a division in 64 bits, whose
+    rounding to 32 is the correctly rounded quotient."""
+    import torch
+
+    class View:
+        def __init__(self, t):
+            self.ptr, self.nbytes = t.data_ptr(), t.numel() * 4
+
+    half = 1 << 23
+    y = torch.empty(2 * half, device="cuda")
+    for exponent in range(-26, 7):
+        bits = torch.arange(half, device="cuda", dtype=torch.int32) + ((127 + exponent) << 23)
+        x = torch.cat([bits.view(torch.float32), -bits.view(torch.float32)])
+        torch.cuda.synchronize()
+        hip.model_aux(View(y), View(x), None, None, mode=5, count=2 * half, width=half)
+        hip.sync()
+        e = torch.exp2(torch.clamp(x.abs() * np.float32(-1.4426950408889634).item(), min=-126.0))
+        inv = (1.0 / (e + 1.0).double()).float()
+        want = x * torch.where(x < 0, e * inv, inv)
+        differ = int((y.view(torch.int32) != want.view(torch.int32)).sum().item())
+        assert differ == 0, (exponent, differ)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("other", [1, 2, 3, 4, 63, 64, 65, 4095, 4096, 4097, 1 << 20, 5000000])
 def test_aux_index_divisors_gpu(hip, orc, other):
     """Whole and split quads of w, divisors around powers of two, the last quad; bit-exact."""

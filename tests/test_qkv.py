@@ -881,15 +881,19 @@ def test_hb_qkv_gemm_parts_equal_gemm_then_post(hip, image, text, n_heads, hd, k
         h.qkv_gemm_parts(*got, parts, pe_dev, pe_rows, k, n_heads, hd, tiles, ws)
     h.sync()
     for which, (g, w) in enumerate(zip(got, want)):
-        a, b = g.read(np.uint16, size), w.read(np.uint16, size)
-        if min(image, text) > 128:
-            assert np.array_equal(a, b), (which, int((a != b).sum()))
-        else:
-            # up to 128 rows the reference product may add k in another order:
-            # one ulp of the fp16 readout, 2^-11 relative, then Q / K values up
-            # to about 4 x 1.5 in fp16, whose own rounding adds as much
-            fa, fb = (v.view(np.float16).astype(np.float32) for v in (a, b))
-            assert np.all(np.abs(fa - fb) <= 2 ** -9 * (1.0 + np.abs(fb))), which
+        # [head][token tile] (Q, K) or [head][column tile][token tile] (V) of 32-token tiles
+        order = (n_heads, tiles, hd * 32) if which < 2 else (n_heads, hd // 32, tiles, 1024)
+        a, b = (np.moveaxis(v.read(np.uint16, size).reshape(order), -2, 0) for v in (g, w))
+        for tokens, t0, t1 in ((image, 0, image // 32), (text, image // 32, tiles - 1)):
+            if tokens > 128:
+                assert np.array_equal(a[t0:t1], b[t0:t1]), (which, tokens, int((a[t0:t1] != b[t0:t1]).sum()))
+            else:
+                # up to 128 rows the reference product may add k in another order:
+                # one ulp of the fp16 readout, 2^-11 relative, then Q / K values up
+                # to about 4 x 1.5 in fp16, whose own rounding adds as much
+                fa, fb = (np.ascontiguousarray(v[t0:t1]).view(np.float16).astype(np.float32) for v in (a, b))
+                assert np.all(np.abs(fa - fb) <= 2 ** -9 * (1.0 + np.abs(fb))), (which, tokens)
+        assert np.all(a[tiles - 1] == 0x1234), which
 
 
 @pytest.mark.gpu
