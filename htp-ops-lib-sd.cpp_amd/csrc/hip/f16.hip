@@ -722,14 +722,14 @@ __device__ inline void splitk_store(hb_f32x4 (&acc)[FM][FN], float *__restrict__
     }
 }
 
-// Split-K form of the ring kernel for up to 128 rows: grid (tiles, splits),
+// Split-K form of the ring kernel (33 to 4095 rows): grid (tiles, splits),
 // split s multiplies k-steps [s*kps, s*kps + kps) of its BM x BN tile (the
 // k loop of f16_gemm_ring on that range) and stores the raw fp32 sums to
 // slice s of the workspace ([mp][n] per slice, rows past m dropped by the
 // buffer bound); f16_skinny_epilogue then adds the slices in order, reads
-// out to fp16 and applies bias and activation.  A tile covers every row, so
-// the fp16 weights are read once, and the splits give the launch enough
-// workgroups.
+// out to fp16 and applies bias and activation.  The splits give the launch
+// enough workgroups; each row of tiles asks for the fp16 weights again (up to
+// 128 rows: once).
 template <int BM, int BN, int WM, int WN, int S>
 __global__ __launch_bounds__(64 * WM *WN) void f16_ring_splitk(float *__restrict__ ws, const int8_t *__restrict__ aimg,
                                                                const int8_t *__restrict__ wpack, int m, int k, int n,
@@ -2298,8 +2298,8 @@ bool wide_fits(int k, int n) {
 // tile's loads), then the 256 x 64 tiles, two of whose workgroups share a CU.
 // The latter against the former, 323 shapes of n 7000-16384: k 256-400 + 10 %,
 // 400-800 + 7 %, 800-1200 + 3.5 %, 1200-2400 between - 8 and + 7 % (+ 0.5 % on
-// average), 2400-2800 - 2 to - 10 %, 4096 - 12 % (us, 212x544x14208 13.1 / 12.1,
-// 231x1728x11232 22.0 / 20.7, 256x4096x14336 47.5 / 56.4).
+// average), 2400-2800 - 2 to - 10 %, 4096 - 5 to - 16 % (us, 212x544x14208 13.1 /
+// 12.1, 231x1728x11232 22.0 / 20.7, 256x4096x14336 40.6 / 42.7).
 constexpr int kStream64Stages = 7, kStream64Depth = 2400;
 
 bool one_row_of_tiles(int m, int k, int n) {

@@ -378,9 +378,12 @@ int hb_qkv_post(uint16_t *d_q, uint16_t *d_k, uint16_t *d_v, const float *d_raw,
  * d_x (tokens x input_dim f32) times the hb_f16_prepack image of the
  * input_dim x 3*n_heads*head_dim weight, with the post-processing of
  * hb_qkv_post applied to each output tile in registers, so the f32 product
- * never reaches HBM.  Results are identical to hb_f16_gemm_ws (mode
- * 0, no bias) followed by hb_qkv_post.  n_heads * head_dim must be a
- * multiple of 128; d_workspace (256-byte aligned) holds
+ * never reaches HBM.  K is never split: results are identical to hb_f16_gemm_ws
+ * (mode 0, no bias) followed by hb_qkv_post where hb_qkv_gemm_unsplit gives 1,
+ * and within the F16 bound of it elsewhere.  d_pe holds the rows that the call
+ * rotates (rope_offset + t for its tokens t while that is below rope_count);
+ * no others are read.  input_dim is below 8388608 (32-bit offsets); n_heads *
+ * head_dim must be a multiple of 128; d_workspace (256-byte aligned) holds
  * hb_qkv_gemm_workspace_bytes(tokens, input_dim) bytes, no state.
  * hb_qkv_gemm_parts does one or two parts (an image and a text half with
  * their own activations, weights, bias and norms, into one packed output) in
